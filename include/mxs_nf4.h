@@ -300,6 +300,11 @@ int mxs_lora_grad_b(const void* ht, int ldt, const void* dy, int M, int N, int r
  * M*K/8. */
 int mxs_keep_pack(const void* keep, int M, int K, void* bits, hipStream_t stream);
 
+/* mxs_keep_pack of n (1..4) byte masks [M, K] in one launch (the projections reading one input
+ * draw a mask each). */
+int mxs_keep_pack_group(int n, const void* const keep[], int M, int K, void* const bits[],
+                        hipStream_t stream);
+
 /* Number of reduction slices (1..4) mxs_lora_h_partials / mxs_lora_dh_partials use for M tokens
  * and a reduction of length Kr: their partials buffer is fp32 [slices][ldt][r]. */
 int mxs_lora_slices(int M, int Kr);

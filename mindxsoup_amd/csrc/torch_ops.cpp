@@ -132,6 +132,41 @@ Tensor keep_mask(const OptTensor& keep, int64_t M, int64_t K, const at::Device& 
   return bits;
 }
 
+// The keep masks of several projections over one input [M, K]: every byte mask packed, all of
+// them in one launch when there are several; undefined where there is none.
+std::vector<Tensor> keep_masks(const std::vector<OptTensor>& keep, int64_t M, int64_t K,
+                               const at::Device& dev) {
+  std::vector<Tensor> out(keep.size());
+  std::vector<size_t> bytes;
+  for (size_t i = 0; i < keep.size(); ++i) {
+    if (!keep[i].has_value() || !keep[i]->defined()) continue;
+    const Tensor& k = *keep[i];
+    const auto t = k.scalar_type();
+    if ((t == at::kByte || t == at::kChar || t == at::kBool) && k.dim() == 2 && k.size(0) == M &&
+        k.size(1) == K && k.device() == dev && !k.is_meta())
+      bytes.push_back(i);
+    else
+      out[i] = keep_mask(keep[i], M, K, dev);  // bits, fake tensors, or refused by name
+  }
+  if (bytes.size() < 2 || bytes.size() > kMaxGroup) {
+    for (size_t i : bytes) out[i] = keep_mask(keep[i], M, K, dev);
+    return out;
+  }
+  std::vector<Tensor> src;
+  std::array<const void*, kMaxGroup> ps{};
+  std::array<void*, kMaxGroup> pb{};
+  for (size_t j = 0; j < bytes.size(); ++j) {
+    src.push_back(keep[bytes[j]]->contiguous());
+    out[bytes[j]] = at::empty({M, (K + 31) / 32}, src[j].options().dtype(at::kInt));
+    ps[j] = src[j].data_ptr();
+    pb[j] = out[bytes[j]].data_ptr();
+  }
+  ok(mxs_keep_pack_group((int)bytes.size(), ps.data(), as_int(M, "M"), as_int(K, "K"), pb.data(),
+                         stream_of(src[0])),
+     "mxs_keep_pack_group");
+  return out;
+}
+
 // keep_mask over the rows of x (a node packs once in its forward and saves the bits).
 OptTensor keep_bits_for(const OptTensor& keep, const Tensor& x2) {
   const Tensor b = keep_mask(keep, x2.size(0), x2.size(1), x2.device());
@@ -1187,7 +1222,12 @@ struct NF4LoraSiblingsFunction : public torch::autograd::Function<NF4LoraSibling
     at::AutoDispatchBelowADInplaceOrView below;
     const size_t n = lora_a.size();
     OptTensorList kbs;
-    for (size_t i = 0; i < keep.size(); ++i) kbs.push_back(keep_bits_for(entry(keep, i), x));
+    {
+      const at::OptionalDeviceGuard guard(at::device_of(x));
+      for (const Tensor& b : keep_masks(entries(keep, keep.size()), x.size(0), x.size(1),
+                                        x.device()))
+        kbs.push_back(b.defined() ? OptTensor(b) : std::nullopt);
+    }
     auto [ys, hts, ats, bts] = fwd.call(x, lora_a, lora_b, packed, absmax8, code, absmax2,
                                         offset, bias, kbs, mask_scale, s, one_gemm, cos, sin,
                                         n_rope);
