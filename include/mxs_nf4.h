@@ -435,6 +435,23 @@ int mxs_nf4_linear_fwd_hp_group_rope(int n, const void* const x[], int M, int K,
                                      const float* sin, int64_t cos_stride_b,
                                      int64_t cos_stride_t, int n_tokens, hipStream_t stream);
 
+/* mxs_nf4_linear_fwd_hp_group (n_rope 0) or its _rope form with a workspace: where
+ * mxs_nf4_linear_fwd_group_workspace_bytes(n, M, N, K, n_rope) is not 0 (many tokens: decoding
+ * each weight once costs less than decoding it per row band) and the workspace (16-byte aligned,
+ * no initial contents needed) holds that many bytes, the weights are decoded to fp16 there and
+ * one plain fp16 GEMM launch computes every output; elsewhere the call is the fused one.  The
+ * same bits either way.  Wide outputs (gate and up) are taken too. */
+int64_t mxs_nf4_linear_fwd_group_workspace_bytes(int n, int M, const int N[], int K, int n_rope);
+int mxs_nf4_linear_fwd_hp_group_ws(int n, const void* const x[], int M, int K, const int N[],
+                                   const void* const packed[], const void* const absmax8[],
+                                   const float* const code[], const float* const absmax2[],
+                                   const float* const offset[], const void* const bias[],
+                                   const float* const lora_hp[], int hp_slices, int ldt,
+                                   const void* const lora_b[], int r, void* const lora_ht[],
+                                   void* const y[], int n_rope, const float* cos,
+                                   const float* sin, int64_t cos_stride_b, int64_t cos_stride_t,
+                                   int n_tokens, void* workspace, hipStream_t stream);
+
 /* 1 when mxs_nf4_linear_bwd_dx_grads_group takes these n (1..4) projections [K -> N[i]] at M
  * tokens: each one mxs_nf4_linear_bwd_grads_fused(M, N[i], K, r) would run as one launch on
  * 128x128 tiles. */
@@ -484,6 +501,19 @@ int mxs_nf4_linear_bwd_dx_grads_sum(int n, const void* const dy[], int M, const 
                                     const void* const ht[], int ldt, const void* x,
                                     float* const da[], float* const db[], void* dx,
                                     hipStream_t stream);
+
+/* mxs_nf4_linear_bwd_dx_grads_sum's dX alone (da and db NULL) from weights decoded once to fp16 in
+ * the workspace (16-byte aligned, no initial contents needed), for the token counts where
+ * mxs_nf4_linear_bwd_dx_sum_workspace_bytes(n, M, N, K, r) is not 0; MXS_ERR_SIZE elsewhere.
+ * The same products in the same order into one fp32 accumulator; with few tiles the reduction is
+ * split and its fp32 planes are added before the one rounding. */
+int64_t mxs_nf4_linear_bwd_dx_sum_workspace_bytes(int n, int M, const int N[], int K, int r);
+int mxs_nf4_linear_bwd_dx_sum(int n, const void* const dy[], int M, const int N[], int K,
+                              const void* const packed[], const void* const absmax8[],
+                              const float* const code[], const float* const absmax2[],
+                              const float* const offset[], const void* const lora_dh[],
+                              const void* const lora_at[], int r, const void* const mask[],
+                              float mask_scale, void* dx, void* workspace, hipStream_t stream);
 
 /* The up projection's forward with the SwiGLU after it (solution/mlp.py:42-43:
  * silu_mul(gate_proj(x), up_proj(x))): mxs_nf4_linear_fwd_hp (lora_hp may be NULL: no LoRA

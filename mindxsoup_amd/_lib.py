@@ -75,6 +75,12 @@ _SIGNATURES = {
                                     P, P],
     "mxs_nf4_linear_fwd_hp_group_rope": [I32, P, I32, I32, P, P, P, P, P, P, P, P, I32, I32, P,
                                          I32, P, P, I32, P, P, I64, I64, I32, P],
+    "mxs_nf4_linear_fwd_group_workspace_bytes": [I32, I32, P, I32, I32],
+    "mxs_nf4_linear_fwd_hp_group_ws": [I32, P, I32, I32, P, P, P, P, P, P, P, P, I32, I32, P,
+                                       I32, P, P, I32, P, P, I64, I64, I32, P, P],
+    "mxs_nf4_linear_bwd_dx_sum_workspace_bytes": [I32, I32, P, I32, I32],
+    "mxs_nf4_linear_bwd_dx_sum": [I32, P, I32, P, I32, P, P, P, P, P, P, P, I32, P, F32, P, P,
+                                  P],
     "mxs_qkv_rope": [P, P, P, P, I64, I64, I32, I32, I32, I32, I32, I32, I32, F32, F32, P],
     "mxs_silu_mul_bwd": [P, P, P, I64, P],
     "mxs_lora_slices": [I32, I32],
@@ -104,6 +110,8 @@ _SIGNATURES = {
 _RESTYPES = {"mxs_nf4_dequant_layer_plan": ctypes.c_int64,
              "mxs_nf4_gemm_workspace_bytes": ctypes.c_int64,
              "mxs_lora_workspace_bytes": ctypes.c_int64,
+             "mxs_nf4_linear_fwd_group_workspace_bytes": ctypes.c_int64,
+             "mxs_nf4_linear_bwd_dx_sum_workspace_bytes": ctypes.c_int64,
              "mxs_nf4_linear_bwd_dx_pair_workspace_bytes": ctypes.c_int64}
 
 

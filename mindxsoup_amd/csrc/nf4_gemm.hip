@@ -17,6 +17,8 @@
 // the input gradient masked by the dropout keep mask), computed before the main loop; the
 // epilogue stores fp16.  With split-K (gridDim.z > 1) each split writes fp32 partials and
 // k_splitk_reduce sums them (split 0 carries bias and LoRA).
+#include <algorithm>
+#include <array>
 #include <atomic>
 #include <functional>
 #include <mutex>
@@ -36,6 +38,7 @@ constexpr int kBK = 64;           // reduction indices per K-step (one NF4 block
 struct GemmArgs {
   const _Float16* A;        // [M, lda]
   int64_t lda;
+  const _Float16* w16;      // dense route: the decoded weight as [Nc, Kr] (W or W^T), else null
   const uint8_t* packed;    // NF4 W [Nw, Kw] (Nw = out_features, Kw = in_features)
   const uint8_t* absmax8;
   const float* code;
@@ -2147,6 +2150,12 @@ __global__ __launch_bounds__(64 * (4 + PW)) void k_nf4_gemm_ws_group(GemmGroup g
                                                      local / g.gx[i]);
 }
 
+}  // namespace mxs
+
+#include "dense_tile.h"
+
+namespace mxs {
+
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool BWD>
 static int launch_cfg(const GemmArgs& a0, int splits, hipStream_t stream) {
   using T = Tile<BM, BN, WAVES_M, WAVES_N, BWD>;
@@ -2326,10 +2335,211 @@ static int check_gemm(bool bwd, const GemmArgs& a) {
   return MXS_OK;
 }
 
+// ---- the dense route (dense_tile.h) -------------------------------------------------------------
+
+// Tile columns and split count of a dense launch.
+struct DensePlan {
+  int bn, splits;
+};
+
+// What the dense route and the fused kernels cost, in microseconds on MI355X (HIP graphs, M = 1024
+// to 8192, the projections' shapes): rounds of tiles over the CUs times a tile's time, which is a
+// K-step's time (power-limited when every CU multiplies) plus what stands alone at its ends.  The
+// route is taken where its estimate is 5 % below the fused kernels'.  Measured / estimated, dense
+// against fused: down_proj forward at 8192 tokens 220 / 228 against 370, at 3001 105 / 104 against
+// 128, at 2048 80 / 79 against 88; its dX (8960 wide) 244 / 247 against 267 at 8192, 68 / 66
+// against 75 at 2048, not taken at 3001 (113 / 129 against 112); 1536 x 1536 at 8192 49 / 47
+// against 66, not taken at 4096 (39 against 39).
+static double fused_tile_us(int cfg, int steps) {
+  switch (cfg) {
+    case 7: return 1.15 * steps + 8.0;             // 256x160
+    case 9: case 11: return 0.87 * steps + 8.0;    // 256x96
+    case 10: return 0.60 * steps + 6.5;            // 128x128
+    default: return 0.41 * steps + 4.7;            // 128x64
+  }
+}
+
+static double dense_tile_us(int bn, int steps) {
+  const double step = bn == 320 ? 1.78 : bn == 256 ? 1.47 : 1.32;
+  return step * steps + 13.0;
+}
+
+static double reduce_us(int splits, int M, int Nc) {
+  return splits > 1 ? (4.0 * splits + 2.0) * M * Nc / 5.4e6 + 2.0 : 0.0;
+}
+
+static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// One GEMM on its fused plan (choose), or a negative number where the dense route is no
+// alternative (outputs narrower than 1024).
+static double fused_us(int M, int Nc, int Kr, bool bwd, bool glu) {
+  int cfg, sp;
+  choose(M, Nc, Kr, bwd, &cfg, &sp);
+  if (cfg < 6) return -1.0;
+  static const int kBM[] = {256, 256, 128, 256, 128, 256, 128};  // cfg 6..12
+  static const int kBN[] = {128, 160, 128, 96, 128, 96, 64};
+  const int64_t tiles = ceil_div(M, kBM[cfg - 6]) * ceil_div(Nc, kBN[cfg - 6]) * sp;
+  const double tail = glu ? 11.3 : 0.0;  // the SwiGLU's gate / up traffic, per round
+  return ceil_div(tiles, cu_count()) *
+             (fused_tile_us(cfg, (int)ceil_div(Kr / kBK, sp)) + tail) +
+         reduce_us(sp, M, Nc);
+}
+
+// The best dense plan for n problems [M, Nc[i]] over `steps` K-steps (sum: one output Nc[0] and
+// all problems' steps together), `values` weight values to decode; its time, or a negative
+// number if there is none.  `bn`: only this tile width (0: any).
+static double dense_us(int M, int n, const int* Nc, int steps, int64_t values, bool sum, bool glu,
+                       int bn, DensePlan* d) {
+  const int cus = cu_count();
+  if (cus <= 0 || M <= 0 || steps <= 0) return -1.0;
+  const int64_t gy = ceil_div(M, kDenseBM);
+  double best = -1.0;
+  for (int w : {320, 256, 192}) {
+    if (bn ? w != bn : (sum && w != 192)) continue;  // summed tiles: 192 (registers)
+    int64_t tiles = 0;
+    for (int i = 0; i < (sum ? 1 : n); i++) tiles += gy * ceil_div(Nc[i], w);
+    for (int sp = 1; sp <= 8; sp++) {
+      if (sp > 1 && (w == 320 || (n > 1 && !sum) || steps / sp < 12)) break;
+      const int per = (int)ceil_div(steps, sp);
+      if (ceil_div(steps, per) != sp) continue;
+      const double t = ceil_div(tiles * sp, cus) *
+                           (dense_tile_us(w, per) + (glu ? 0.09 * w : 0.0)) +
+                       reduce_us(sp, M, Nc[0]) + 2.53 * values / 4.2e6 + 1.5;
+      if (best < 0 || t < best) {
+        best = t;
+        d->bn = w;
+        d->splits = sp;
+      }
+    }
+  }
+  return best;
+}
+
+static bool dense_plan(int M, int Nc, int Kr, bool bwd, bool glu, DensePlan* d) {
+  const double f = fused_us(M, Nc, Kr, bwd, glu);
+  if (f < 0) return false;
+  const double t = dense_us(M, 1, &Nc, Kr / kBK, (int64_t)Nc * Kr, false, glu, 0, d);
+  return t > 0 && t < 0.95 * f;
+}
+
+// The copies' 32-bit offsets (a tile's rows of either operand) and whole keep words per tile.
+static bool dense_takes(int M, int Nc, int Kr) {
+  return M > 0 && Nc > 0 && Kr > 0 && Kr % kBK == 0 && Nc % 64 == 0 &&
+         (int64_t)320 * Kr * 2 < (int64_t(1) << 32) && (int64_t)Nc * Kr < (int64_t(1) << 40);
+}
+
+static int64_t w16_bytes(int Nc, int Kr) { return (int64_t)Nc * Kr * 2; }
+
+// Decode every problem's weight into its w16.
+static int launch_w16(bool bwd, const GemmArgs* p, int n, hipStream_t stream) {
+  W16Group g{};
+  g.n = n;
+  int64_t total = 0;
+  for (int i = 0; i < n; i++) {
+    const int N = bwd ? p[i].Kr : p[i].Nc, K = p[i].Kw;
+    g.p[i] = {reinterpret_cast<const uint32_t*>(p[i].packed), p[i].absmax8, p[i].code,
+              p[i].absmax2, p[i].offset, const_cast<_Float16*>(p[i].w16), N, K};
+    g.start[i] = (int)total;
+    total += bwd ? (N / kW16TR) * ceil_div(K, kW16TC)
+                 : ceil_div((int64_t)N * K / 8, kW16Chunks);
+    if (total > 0x7fffffff) return MXS_ERR_SIZE;
+  }
+  g.start[n] = (int)total;
+  if (bwd) hipLaunchKernelGGL(k_w16_decode<true>, dim3(total), dim3(256), 0, stream, g);
+  else hipLaunchKernelGGL(k_w16_decode<false>, dim3(total), dim3(256), 0, stream, g);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? MXS_OK : (int)e;
+}
+
+template <int BN, bool BWD, bool GLU, int NSUM, bool ROPE>
+static int launch_dense_tile(const DenseGroup& g, int tiles, int splits, hipStream_t stream) {
+  const void* fn = reinterpret_cast<const void*>(&k_dense_gemm<BN, BWD, GLU, NSUM, ROPE>);
+  constexpr int lds = dense_lds_bytes<BN>();
+  static bool lds_set = false;  // idempotent attribute; a benign race between threads
+  if (!lds_set) {
+    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return (int)e;
+    lds_set = true;
+  }
+  hipLaunchKernelGGL((k_dense_gemm<BN, BWD, GLU, NSUM, ROPE>), dim3(tiles, 1, splits),
+                     dim3(kDenseNT), lds, stream, g);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? MXS_OK : (int)e;
+}
+
+// n problems (checked by check_gemm and dense_takes) on plan d: the weights decoded into the
+// workspace, then one GEMM launch (forward: each its own output, rope_cos rotated; backward: one
+// problem, or `sum` into problem 0's output) and, where `reduce`, the splits' reduce.  ws: the
+// decoded weights, then the partial planes.  *planes (optional): where those are.
+static int launch_dense(bool bwd, const GemmArgs* probs, int n, bool sum, const DensePlan& d,
+                        void* ws, bool reduce, float** planes, hipStream_t stream) {
+  if (n < 1 || n > kMaxGemmGroup || (sum && (n > kMaxSum || !bwd)) || (bwd && !sum && n > 1) ||
+      !ws || (uintptr_t)ws % 16)
+    return MXS_ERR_ARG;
+  DenseGroup g{};
+  g.n = n;
+  g.gy = (int)ceil_div(probs[0].M, kDenseBM);
+  char* w = static_cast<char*>(ws);
+  int steps = 0;
+  int64_t tiles = 0;
+  bool rope = false;
+  for (int i = 0; i < n; i++) {
+    GemmArgs a = probs[i];
+    a.w16 = reinterpret_cast<const _Float16*>(w);
+    w += w16_bytes(a.Nc, a.Kr);
+    a.zf = 0;
+    a.unsplit = 0;
+    a.cols_blocks = 0;
+    rope = rope || a.rope_cos;
+    steps = sum ? steps + a.Kr / kBK : a.Kr / kBK;
+    g.start[i] = (int)tiles;
+    if (!sum || i == 0) tiles += g.gy * ceil_div(a.Nc, d.bn);
+    g.p[i] = a;
+  }
+  g.start[n] = (int)tiles;
+  if (tiles > 0x7fffffff || (rope && d.bn != 256)) return MXS_ERR_SIZE;
+  const int per = (int)ceil_div(steps, d.splits);
+  const int splits = (int)ceil_div(steps, per);
+  if (splits > 1 && (d.bn > 256 || (n > 1 && !sum))) return MXS_ERR_ARG;
+  for (int i = 0; i < n; i++) {
+    g.p[i].ws = reinterpret_cast<float*>(w);
+    g.p[i].steps_per_split = per;
+  }
+  if (planes) *planes = reinterpret_cast<float*>(w);
+  int rc = launch_w16(bwd, g.p, n, stream);
+  if (rc != MXS_OK) return rc;
+  const int t = (int)tiles;
+  const bool glu = probs[0].glu == 2;
+  if (sum)
+    rc = launch_dense_tile<192, true, false, kMaxSum, false>(g, t, splits, stream);
+  else if (rope)
+    rc = launch_dense_tile<256, false, false, 1, true>(g, t, splits, stream);
+  else if (d.bn == 320)
+    rc = !bwd ? launch_dense_tile<320, false, false, 1, false>(g, t, splits, stream)
+        : glu ? launch_dense_tile<320, true, true, 1, false>(g, t, splits, stream)
+              : launch_dense_tile<320, true, false, 1, false>(g, t, splits, stream);
+  else if (d.bn == 256)
+    rc = !bwd ? launch_dense_tile<256, false, false, 1, false>(g, t, splits, stream)
+        : glu ? launch_dense_tile<256, true, true, 1, false>(g, t, splits, stream)
+              : launch_dense_tile<256, true, false, 1, false>(g, t, splits, stream);
+  else
+    rc = !bwd ? launch_dense_tile<192, false, false, 1, false>(g, t, splits, stream)
+        : glu ? launch_dense_tile<192, true, true, 1, false>(g, t, splits, stream)
+              : launch_dense_tile<192, true, false, 1, false>(g, t, splits, stream);
+  if (rc != MXS_OK) return rc;
+  return splits > 1 && reduce ? launch_reduce(g.p[0], splits, stream) : MXS_OK;
+}
+
 static int gemm_entry(bool bwd, const GemmArgs& a, int cfg, int splits, hipStream_t stream) {
   const int c = check_gemm(bwd, a);
   if (c != MXS_OK) return c == 1 ? MXS_OK : c;
-  if (cfg < 0) choose(a.M, a.Nc, a.Kr, bwd, &cfg, &splits);
+  if (cfg < 0) {
+    DensePlan d;
+    if (a.ws && (uintptr_t)a.ws % 16 == 0 && a.glu != 1 && a.cols_blocks == 0 &&
+        dense_takes(a.M, a.Nc, a.Kr) && dense_plan(a.M, a.Nc, a.Kr, bwd, a.glu == 2, &d))
+      return launch_dense(bwd, &a, 1, false, d, a.ws, true, nullptr, stream);
+    choose(a.M, a.Nc, a.Kr, bwd, &cfg, &splits);
+  }
   if (cfg >= kNumCfg || cfg == 5) return MXS_ERR_ARG;
   return bwd ? launch_by_id<true>(cfg, a, splits, stream)
              : launch_by_id<false>(cfg, a, splits, stream);
@@ -2753,6 +2963,77 @@ static bool pair_plan_ok(int M, int N0, int N1, int K) {
   return true;
 }
 
+// Dense alternatives of the launches that take several problems.
+static bool dense_takes_all(int n, int M, const int* N, int K, bool bwd) {
+  for (int i = 0; i < n; i++)
+    if (!(bwd ? dense_takes(M, K, N[i]) : dense_takes(M, N[i], K))) return false;
+  return true;
+}
+
+static int64_t weight_values(int n, const int* N, int K) {
+  int64_t v = 0;
+  for (int i = 0; i < n; i++) v += (int64_t)N[i] * K;
+  return v;
+}
+
+// Workspace of n summed problems [K <- N[i]] on plan d.
+static int64_t dense_sum_bytes(int n, int M, const int* N, int K, const DensePlan& d) {
+  const int64_t planes = d.splits > 1 ? (int64_t)d.splits * M * K * 4 : 0;
+  return 2 * weight_values(n, N, K) + planes;
+}
+
+// The gate / up pair's summed dX (against its split-K launch on 256x96 tiles).  Measured at 8192
+// tokens: 469 us and 19 us of decode against 613 us and a reduce of four planes; at 3001 tokens
+// 192 + 17 (and a reduce of two planes instead of four) against 212.
+static bool dense_pair_plan(int M, const int N[2], int K, DensePlan* d) {
+  if (cu_count() <= 0 || !dense_takes_all(2, M, N, K, true)) return false;
+  int steps = 0, longest = 0;
+  for (int i = 0; i < 2; i++) {
+    steps += N[i] / kBK;
+    longest = std::max(longest, N[i] / kBK);
+  }
+  const double f = ceil_div(ceil_div(M, 256) * ceil_div(K, 96) * 2 * kPairSplits, cu_count()) *
+                       fused_tile_us(11, (int)ceil_div(longest, kPairSplits)) +
+                   reduce_us(2 * kPairSplits, M, K);
+  const double t = dense_us(M, 2, &K, steps, weight_values(2, N, K), true, false, 0, d);
+  return t > 0 && t < 0.95 * f;
+}
+
+// q, k and v's summed dX without their gradients (against one launch of 128x128 tiles): 84 us
+// and 5 us of decode against 110 at 8192 tokens.
+static bool dense_sum_plan(int n, int M, const int* N, int K, DensePlan* d) {
+  if (cu_count() <= 0 || n < 2 || n > kMaxSum || !dense_takes_all(n, M, N, K, true)) return false;
+  int steps = 0;
+  for (int i = 0; i < n; i++) steps += N[i] / kBK;
+  const double f = ceil_div(ceil_div(M, 128) * ceil_div(K, 128), cu_count()) *
+                   (fused_tile_us(10, steps) + 8.0);
+  const double t = dense_us(M, n, &K, steps, weight_values(n, N, K), true, false, 0, d);
+  return t > 0 && t < 0.95 * f;
+}
+
+// Several forwards over one input in one launch: q, k and v (against 128x128 tiles; 70 us, rotated,
+// and 5 us of decode against 108 at 8192 tokens), or wide outputs (gate and up, against 256x160
+// tiles of which a mixed launch saves 5 %; 448 + 15 against 527 us at 8192, 164 + 14 against 209
+// at 3001).
+static bool dense_group_plan(int n, int M, const int* N, int K, bool rope, DensePlan* d) {
+  if (cu_count() <= 0 || n < 1 || n > kMaxGemmGroup || !dense_takes_all(n, M, N, K, false))
+    return false;
+  bool wide = true;
+  int64_t tiles128 = 0, tiles160 = 0;
+  for (int i = 0; i < n; i++) {
+    wide = wide && N[i] >= 4096;
+    tiles128 += ceil_div(M, 128) * ceil_div(N[i], 128);
+    tiles160 += ceil_div(M, 256) * ceil_div(N[i], 160);
+  }
+  const int steps = K / kBK;
+  const double f = wide && !rope
+      ? 0.95 * ceil_div(tiles160, cu_count()) * fused_tile_us(7, steps)
+      : ceil_div(tiles128, cu_count()) * (fused_tile_us(10, steps) + (rope ? 5.5 : 0.0));
+  const double t = dense_us(M, n, N, steps, weight_values(n, N, K), false, false, rope ? 256 : 0,
+                            d);
+  return t > 0 && t < 0.95 * f;
+}
+
 // The arguments of a dX GEMM whose launch also computes the LoRA gradients (its workgroups past
 // the tiles): the gradients' checks (mxs_lora_grads); the GEMM's follow in check_gemm.
 static int dx_grads_args(const void* dy, int M, int N, int K, const void* packed,
@@ -2859,9 +3140,19 @@ using namespace mxs;
 
 // Split-K workspace: one fp32 partial plane per split.
 int64_t mxs_nf4_gemm_workspace_bytes(int M, int Nc, int Kr, int cfg, int splits) {
-  if (cfg < 0) choose(M, Nc, Kr, false, &cfg, &splits);  // both directions split alike
-  if (splits <= 1) return 0;
-  return (int64_t)splits * M * Nc * (int64_t)sizeof(float);
+  int64_t dense = 0;
+  if (cfg < 0) {
+    if (dense_takes(M, Nc, Kr))
+      for (int v = 0; v < 3; v++) {  // forward, backward, backward with the SwiGLU adjoint
+        DensePlan d;
+        if (!dense_plan(M, Nc, Kr, v > 0, v > 1, &d)) continue;
+        const int64_t planes = d.splits > 1 ? (int64_t)d.splits * M * Nc * 4 : 0;
+        dense = std::max(dense, w16_bytes(Nc, Kr) + planes);
+      }
+    choose(M, Nc, Kr, false, &cfg, &splits);  // both directions split alike
+  }
+  if (splits <= 1) return dense;
+  return std::max(dense, (int64_t)splits * M * Nc * (int64_t)sizeof(float));
 }
 
 static void set_workspace(GemmArgs& a, void* workspace) {
@@ -3147,6 +3438,44 @@ int mxs_nf4_linear_bwd_dx_grads_sum(int n, const void* const dy[], int M, const 
   return bn == 64 ? launch_ws_sum<64>(probs, n, stream) : launch_ws_sum<128>(probs, n, stream);
 }
 
+int64_t mxs_nf4_linear_bwd_dx_sum_workspace_bytes(int n, int M, const int N[], int K, int r) {
+  int bn, nw;
+  DensePlan d;
+  if (!N || !dx_grads_sum_ok(n, M, N, K, r, false, &bn, &nw) || !dense_sum_plan(n, M, N, K, &d))
+    return 0;
+  return dense_sum_bytes(n, M, N, K, d);
+}
+
+int mxs_nf4_linear_bwd_dx_sum(int n, const void* const dy[], int M, const int N[], int K,
+                              const void* const packed[], const void* const absmax8[],
+                              const float* const code[], const float* const absmax2[],
+                              const float* const offset[], const void* const lora_dh[],
+                              const void* const lora_at[], int r, const void* const mask[],
+                              float mask_scale, void* dx, void* workspace, hipStream_t stream) {
+  if (n < 2 || n > kMaxSum || !dy || !N || !packed || !absmax8 || !code || !absmax2 || !offset ||
+      !lora_dh || !lora_at || !dx || !workspace)
+    return MXS_ERR_ARG;
+  int bn, nw;
+  DensePlan d;
+  if (!dx_grads_sum_ok(n, M, N, K, r, false, &bn, &nw) || !dense_sum_plan(n, M, N, K, &d))
+    return MXS_ERR_SIZE;
+  GemmArgs probs[kMaxSum];
+  const bool masked = mask && mask[0];
+  for (int i = 0; i < n; i++) {
+    const void* mk = mask ? mask[i] : nullptr;
+    if (!lora_dh[i] || !lora_at[i] || (mk != nullptr) != masked) return MXS_ERR_ARG;
+    // the gradients' operands are stand-ins (the 16-byte aligned dY) that nothing reads
+    int e = dx_grads_args(dy[i], M, N[i], K, packed[i], absmax8[i], code[i], absmax2[i],
+                          offset[i], lora_dh[i], lora_at[i], r, mk, mask_scale, dy[i], dy[i],
+                          (M + 7) / 8 * 8, dy[i], nullptr, nullptr, dx, 0, probs[i]);
+    if (e != MXS_OK) return e;
+    probs[i].cols_blocks = 0;
+    e = check_gemm(true, probs[i]);
+    if (e != MXS_OK) return e == 1 ? MXS_ERR_SIZE : e;
+  }
+  return launch_dense(true, probs, n, true, d, workspace, true, nullptr, stream);
+}
+
 int mxs_nf4_linear_fwd_hp(const void* x, int M, int K, int N, const void* packed,
                           const void* absmax8, const float* code, const float* absmax2,
                           const float* offset, const void* bias, const float* lora_hp,
@@ -3270,7 +3599,10 @@ int mxs_nf4_linear_bwd_dx_pair_ok(int M, int N0, int N1, int K) {
 
 int64_t mxs_nf4_linear_bwd_dx_pair_workspace_bytes(int M, int N0, int N1, int K) {
   if (!pair_plan_ok(M, N0, N1, K)) return 0;
-  return (int64_t)2 * kPairSplits * M * K * (int64_t)sizeof(float);
+  const int64_t fused = (int64_t)2 * kPairSplits * M * K * (int64_t)sizeof(float);
+  const int N[2] = {N0, N1};
+  DensePlan d;
+  return dense_pair_plan(M, N, K, &d) ? std::max(fused, dense_sum_bytes(2, M, N, K, d)) : fused;
 }
 
 int mxs_nf4_linear_bwd_dx_hp_pair(const void* const dy[2], int M, const int N[2], int K,
@@ -3286,6 +3618,9 @@ int mxs_nf4_linear_bwd_dx_hp_pair(const void* const dy[2], int M, const int N[2]
                              hp_slices, ldt, lora_at, r, mask, mask_scale, lora_dht, dx,
                              workspace, p);
   if (c != MXS_OK) return c == 1 ? MXS_OK : c;
+  DensePlan d;
+  if (dense_pair_plan(M, N, K, &d) && (uintptr_t)workspace % 16 == 0)
+    return launch_dense(true, p, 2, true, d, workspace, true, nullptr, stream);
   return launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], kPairSplits, stream);
 }
 
@@ -3320,11 +3655,24 @@ int mxs_nf4_linear_bwd_dx_hp_pair_grads(
     if (e != MXS_OK) return e;
     if (cols_cpl(K + N[i]) != cpl) return MXS_ERR_SIZE;
   }
-  const int e = launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], kPairSplits, stream, false);
-  if (e != MXS_OK) return e;
-  if (cpl == 8) return reduce_cols_launch<8>(p[0], 2 * kPairSplits, g, M, ldt, r, stream);
-  if (cpl == 4) return reduce_cols_launch<4>(p[0], 2 * kPairSplits, g, M, ldt, r, stream);
-  return reduce_cols_launch<2>(p[0], 2 * kPairSplits, g, M, ldt, r, stream);
+  int planes = 2 * kPairSplits;
+  DensePlan d;
+  if (dense_pair_plan(M, N, K, &d) && (uintptr_t)workspace % 16 == 0) {
+    const int e = launch_dense(true, p, 2, true, d, workspace, false, &p[0].ws, stream);
+    if (e != MXS_OK) return e;
+    planes = d.splits;
+    if (planes == 1)  // dX is complete: the gradients alone
+      return mxs_lora_grads_group(2, lora_dht, ht, ldt, std::array<const void*, 2>{x, x}.data(),
+                                  dy, M, std::array<int, 2>{K, K}.data(), N, r, mask, mask_scale,
+                                  da, db, stream);
+  } else {
+    const int e =
+        launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], kPairSplits, stream, false);
+    if (e != MXS_OK) return e;
+  }
+  if (cpl == 8) return reduce_cols_launch<8>(p[0], planes, g, M, ldt, r, stream);
+  if (cpl == 4) return reduce_cols_launch<4>(p[0], planes, g, M, ldt, r, stream);
+  return reduce_cols_launch<2>(p[0], planes, g, M, ldt, r, stream);
 }
 
 // The rotation the grouped forward may apply to its first n_rope problems (attention's q / k).
@@ -3342,7 +3690,8 @@ static int fwd_hp_group(int n, const void* const x[], int M, int K, const int N[
                         const float* const offset[], const void* const bias[],
                         const float* const lora_hp[], int hp_slices, int ldt,
                         const void* const lora_b[], int r, void* const lora_ht[],
-                        void* const y[], const RopeSpec& rs, hipStream_t stream) {
+                        void* const y[], const RopeSpec& rs, void* workspace,
+                        hipStream_t stream) {
   if (n < 1 || n > kMaxGemmGroup || !x || !N || !packed || !absmax8 || !code || !absmax2 ||
       !offset || !y || rs.n_rope < 0 || rs.n_rope > n)
     return MXS_ERR_ARG;
@@ -3395,6 +3744,9 @@ static int fwd_hp_group(int n, const void* const x[], int M, int K, const int N[
     probs[live++] = a;
   }
   if (live == 0) return MXS_OK;
+  DensePlan d;
+  if (workspace && live == n && dense_group_plan(n, M, N, K, rs.n_rope > 0, &d))
+    return launch_dense(false, probs, n, false, d, workspace, true, nullptr, stream);
   // 128x64 tiles when every problem's tiles together fit the CUs in one round (q, k and v at
   // 1024 tokens: 192 + 32 + 32 = 256 tiles), as the planner does for one problem; else 128x128.
   // With the rotation the 128x64 tiles take 4 x 1 consumer waves (each wave's two 32-column
@@ -3419,7 +3771,7 @@ int mxs_nf4_linear_fwd_hp_group(int n, const void* const x[], int M, int K, cons
                                 const void* const lora_b[], int r, void* const lora_ht[],
                                 void* const y[], hipStream_t stream) {
   return fwd_hp_group(n, x, M, K, N, packed, absmax8, code, absmax2, offset, bias, lora_hp,
-                      hp_slices, ldt, lora_b, r, lora_ht, y, RopeSpec{}, stream);
+                      hp_slices, ldt, lora_b, r, lora_ht, y, RopeSpec{}, nullptr, stream);
 }
 
 int mxs_nf4_linear_fwd_hp_group_rope(int n, const void* const x[], int M, int K, const int N[],
@@ -3434,7 +3786,29 @@ int mxs_nf4_linear_fwd_hp_group_rope(int n, const void* const x[], int M, int K,
   if (n_rope < 1) return MXS_ERR_ARG;
   const RopeSpec rs{n_rope, cos, sin, cos_stride_b, cos_stride_t, n_tokens};
   return fwd_hp_group(n, x, M, K, N, packed, absmax8, code, absmax2, offset, bias, lora_hp,
-                      hp_slices, ldt, lora_b, r, lora_ht, y, rs, stream);
+                      hp_slices, ldt, lora_b, r, lora_ht, y, rs, nullptr, stream);
+}
+
+int64_t mxs_nf4_linear_fwd_group_workspace_bytes(int n, int M, const int N[], int K, int n_rope) {
+  DensePlan d;
+  if (!N || M <= 0 || !dense_group_plan(n, M, N, K, n_rope > 0, &d)) return 0;
+  return 2 * weight_values(n, N, K);
+}
+
+int mxs_nf4_linear_fwd_hp_group_ws(int n, const void* const x[], int M, int K, const int N[],
+                                   const void* const packed[], const void* const absmax8[],
+                                   const float* const code[], const float* const absmax2[],
+                                   const float* const offset[], const void* const bias[],
+                                   const float* const lora_hp[], int hp_slices, int ldt,
+                                   const void* const lora_b[], int r, void* const lora_ht[],
+                                   void* const y[], int n_rope, const float* cos,
+                                   const float* sin, int64_t cos_stride_b, int64_t cos_stride_t,
+                                   int n_tokens, void* workspace, hipStream_t stream) {
+  if (!workspace || n_rope < 0) return MXS_ERR_ARG;
+  if ((uintptr_t)workspace % 16) return MXS_ERR_ALIGN;
+  const RopeSpec rs{n_rope, cos, sin, cos_stride_b, cos_stride_t, n_tokens};
+  return fwd_hp_group(n, x, M, K, N, packed, absmax8, code, absmax2, offset, bias, lora_hp,
+                      hp_slices, ldt, lora_b, r, lora_ht, y, rs, workspace, stream);
 }
 
 int mxs_nf4_linear_glu_fused(int M, int N, int K, int bwd) {

@@ -498,7 +498,19 @@ Lists4 fwd_impl(const Tensor& x, TensorList lora_a, TensorList lora_b, TensorLis
     p_y[i] = ys[i].data_ptr();
     p_ht[i] = hts[i].data_ptr();
   }
-  if (one_gemm && rope.n_rope > 0) {
+  // many tokens: every weight decoded once into a workspace, then one fp16 GEMM launch
+  const bool pair = !one_gemm && n == 2 && mxs_nf4_linear_fwd_pair_ok(m, Ns[0], Ns[1], k);
+  const int64_t group_bytes = one_gemm || pair
+      ? mxs_nf4_linear_fwd_group_workspace_bytes((int)n, m, Ns.data(), k, rope.n_rope) : 0;
+  if (group_bytes > 0) {
+    const Tensor ws = workspace(group_bytes, xc);
+    ok(mxs_nf4_linear_fwd_hp_group_ws(
+           (int)n, xs.data(), m, k, Ns.data(), p_packed.data(), p_a8.data(), p_code.data(),
+           p_a2.data(), p_off.data(), pbias.data(), p_hp.data(), S, (int)ldt, pb.data(), rr,
+           p_ht.data(), p_y.data(), rope.n_rope, rope.cos, rope.sin, rope.cs_b, rope.cs_t,
+           rope.T, ptr(ws), st),
+       "mxs_nf4_linear_fwd_hp_group_ws");
+  } else if (one_gemm && rope.n_rope > 0) {
     ok(mxs_nf4_linear_fwd_hp_group_rope(
            (int)n, xs.data(), m, k, Ns.data(), p_packed.data(), p_a8.data(), p_code.data(),
            p_a2.data(), p_off.data(), pbias.data(), p_hp.data(), S, (int)ldt, pb.data(), rr,
@@ -511,7 +523,7 @@ Lists4 fwd_impl(const Tensor& x, TensorList lora_a, TensorList lora_b, TensorLis
                                    pbias.data(), p_hp.data(), S, (int)ldt, pb.data(), rr,
                                    p_ht.data(), p_y.data(), st),
        "mxs_nf4_linear_fwd_hp_group");
-  } else if (n == 2 && mxs_nf4_linear_fwd_pair_ok(m, Ns[0], Ns[1], k)) {
+  } else if (pair) {
     // gate and up: one launch, grid z selects the projection (the bits of two launches)
     ok(mxs_nf4_linear_fwd_hp_pair(xc.data_ptr(), m, k, Ns.data(), p_packed.data(), p_a8.data(),
                                   p_code.data(), p_a2.data(), p_off.data(), pbias.data(),
@@ -794,13 +806,23 @@ Lists3 lora_bwd_group_cuda(TensorList dy, const Tensor& x, const OptTensorList& 
                            pdht.data(), st),
          "mxs_lora_dh_group");
       dxs[0] = at::empty({M, K}, f16);
-      ok(mxs_nf4_linear_bwd_dx_grads_sum((int)n, pdy.data(), M, Ns.data(), K, pk.data(),
-                                         pa8.data(), pc.data(), pa2.data(), po.data(),
-                                         pdhc.data(), pat.data(), r, pm.data(), ms, pdhtc.data(),
-                                         pht.data(), ldt, o[0].x.data_ptr(),
-                                         fused ? pda.data() : nullptr,
-                                         fused ? pdb.data() : nullptr, dxs[0].data_ptr(), st),
-         "mxs_nf4_linear_bwd_dx_grads_sum");
+      const int64_t sum_bytes = fused ? 0
+          : mxs_nf4_linear_bwd_dx_sum_workspace_bytes((int)n, M, Ns.data(), K, r);
+      if (sum_bytes > 0) {  // many tokens: the weights decoded once, then one fp16 GEMM launch
+        const Tensor sws = workspace(sum_bytes, o[0].x);
+        ok(mxs_nf4_linear_bwd_dx_sum((int)n, pdy.data(), M, Ns.data(), K, pk.data(), pa8.data(),
+                                     pc.data(), pa2.data(), po.data(), pdhc.data(), pat.data(),
+                                     r, pm.data(), ms, dxs[0].data_ptr(), ptr(sws), st),
+           "mxs_nf4_linear_bwd_dx_sum");
+      } else {
+        ok(mxs_nf4_linear_bwd_dx_grads_sum((int)n, pdy.data(), M, Ns.data(), K, pk.data(),
+                                           pa8.data(), pc.data(), pa2.data(), po.data(),
+                                           pdhc.data(), pat.data(), r, pm.data(), ms,
+                                           pdhtc.data(), pht.data(), ldt, o[0].x.data_ptr(),
+                                           fused ? pda.data() : nullptr,
+                                           fused ? pdb.data() : nullptr, dxs[0].data_ptr(), st),
+           "mxs_nf4_linear_bwd_dx_grads_sum");
+      }
       if (!fused) {
         std::vector<bool> done(n, false);
         for (size_t i = 0; i < n; ++i) {

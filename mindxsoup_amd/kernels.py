@@ -314,6 +314,18 @@ def nf4_linear_bwd_dx_grads_sum(dys, packeds, states, dhs, ats, dhts, hts, x2d, 
     da = [torch.empty((r, K), dtype=torch.float32, device=dev) for _ in dys] if grads else None
     db = [torch.empty((nn_, r), dtype=torch.float32, device=dev) for nn_ in Ns] if grads else None
     masks = [keep_bits(m, M, K) for m in masks]
+    nbytes = 0 if grads else int(_lib.lib().mxs_nf4_linear_bwd_dx_sum_workspace_bytes(
+        n, M, _int_array(Ns), K, r))
+    if nbytes:  # many tokens: the weights decoded once, then one fp16 GEMM launch
+        ws = new_workspace(nbytes, dev)
+        _lib.call("mxs_nf4_linear_bwd_dx_sum", n, _ptr_array(dys), M, _int_array(Ns), K,
+                  _ptr_array(packeds), _ptr_array([st.absmax for st in states]),
+                  _ptr_array([st.state2.code for st in states]),
+                  _ptr_array([st.state2.absmax for st in states]),
+                  _ptr_array([st.offset for st in states]), _ptr_array([_c(t) for t in dhs]),
+                  _ptr_array([_c(t) for t in ats]), r, _ptr_array(masks), float(mask_scale),
+                  _lib.ptr(dx), _lib.ptr(ws), _lib.stream_of(dev))
+        return dx, None
     _lib.call("mxs_nf4_linear_bwd_dx_grads_sum", n, _ptr_array(dys), M, _int_array(Ns), K,
               _ptr_array(packeds), _ptr_array([st.absmax for st in states]),
               _ptr_array([st.state2.code for st in states]),
@@ -545,17 +557,30 @@ def nf4_linear_fwd_hp_group(x2ds, packeds, states, lora_hps=None, lora_bs=None, 
             _ptr_array([st.state2.absmax for st in states]),
             _ptr_array([st.offset for st in states]), _ptr_array(bias16), _ptr_array(hps), S,
             ldt, _ptr_array(b16), r, _ptr_array(hts), _ptr_array(ys))
-    if rope is None:
-        _lib.call("mxs_nf4_linear_fwd_hp_group", *args, _lib.stream_of(dev))
-    else:
+    rotation = (0, None, None, 0, 0, 0)
+    if rope is not None:
         n_rope, cos, sin = rope
         cs_b, cs_t, T = rope_spec(n_rope, cos, sin, M)
         if n_rope > n or any(st.shape[0] % 128 for st in states[:n_rope]) \
                 or cos.device != dev or sin.device != dev:
             raise ValueError("rotated outputs: whole 128-column heads on the input's device")
-        _lib.call("mxs_nf4_linear_fwd_hp_group_rope", *args, n_rope, _lib.ptr(cos),
-                  _lib.ptr(sin), cs_b, cs_t, T, _lib.stream_of(dev))
+        rotation = (n_rope, _lib.ptr(cos), _lib.ptr(sin), cs_b, cs_t, T)
+    nbytes = _group_workspace_bytes(M, [st.shape[0] for st in states], K, rotation[0])
+    if nbytes:  # many tokens: every weight decoded once, then one fp16 GEMM launch
+        ws = new_workspace(nbytes, dev)
+        _lib.call("mxs_nf4_linear_fwd_hp_group_ws", *args, *rotation, _lib.ptr(ws),
+                  _lib.stream_of(dev))
+    elif rope is None:
+        _lib.call("mxs_nf4_linear_fwd_hp_group", *args, _lib.stream_of(dev))
+    else:
+        _lib.call("mxs_nf4_linear_fwd_hp_group_rope", *args, *rotation, _lib.stream_of(dev))
     return list(zip(ys, hts))
+
+
+def _group_workspace_bytes(M, Ns, K, n_rope=0):
+    """Bytes of the grouped forward's workspace (0: it takes the fused kernels)."""
+    return int(_lib.lib().mxs_nf4_linear_fwd_group_workspace_bytes(len(Ns), M, _int_array(Ns), K,
+                                                                  n_rope))
 
 
 def nf4_linear_bwd_dx_hp(dy2d, packed, state, lora_dhp, lora_at, mask=None, mask_scale=1.0,
@@ -609,6 +634,19 @@ def nf4_linear_fwd_hp_pair(x2d, packeds, states, lora_hps, lora_bs, biases=None)
         check_nf4_operands(pk, st, dev)
     ys = [torch.empty((M, n), dtype=torch.float16, device=dev) for n in (n0, n1)]
     hts = [torch.empty((r, ldt), dtype=torch.float16, device=dev) for _ in range(2)]
+    nbytes = _group_workspace_bytes(M, [n0, n1], k)
+    if nbytes:  # many tokens: both weights decoded once, then one fp16 GEMM launch
+        ws = new_workspace(nbytes, dev)
+        _lib.call("mxs_nf4_linear_fwd_hp_group_ws", 2, _ptr_array([x2d, x2d]), M, k,
+                  _int_array([n0, n1]), _ptr_array(packeds),
+                  _ptr_array([st.absmax for st in states]),
+                  _ptr_array([st.state2.code for st in states]),
+                  _ptr_array([st.state2.absmax for st in states]),
+                  _ptr_array([st.offset for st in states]), _ptr_array(biases),
+                  _ptr_array([_c(h) for h in lora_hps]), S, ldt,
+                  _ptr_array([_c(b) for b in lora_bs]), r, _ptr_array(hts), _ptr_array(ys), 0,
+                  None, None, 0, 0, 0, _lib.ptr(ws), _lib.stream_of(dev))
+        return list(zip(ys, hts))
     _lib.call("mxs_nf4_linear_fwd_hp_pair", _lib.ptr(x2d), M, k, _int_array([n0, n1]),
               _ptr_array(packeds), _ptr_array([st.absmax for st in states]),
               _ptr_array([st.state2.code for st in states]),
