@@ -66,6 +66,7 @@ struct RowsArgs {
   _Float16* bt;
   float* ws;              // fp32 partials [slices][ldt][r], times s (sliced or partial mode)
   int partial_out;        // write the partials even for one slice; no final fp16 outputs
+  int slices;             // reduction slices of a launch of its own (k_lora_rows)
   // fp32 LoRA weights (the rows kernel's W32 form): R32 [r, K] and B32 [N, r] are read in place
   // of R / B and rounded to fp16 (nearest even) where they are used, so the results are those of
   // R and B cast first; b16 (optional) receives that fp16 copy of B [N, r].
@@ -85,6 +86,39 @@ __device__ __forceinline__ half8_t f32x8_to_f16(const float* p) {
     h[4 + e] = (_Float16)hi[e];
   }
   return h;
+}
+
+// Side outputs, spread over n_wg workgroups of which this is wg: R^T [K, r], B^T [r, N] and (W32)
+// fp16 B [N, r].
+template <bool W32>
+__device__ __forceinline__ void rows_side(const RowsArgs& a, int wg, int n_wg) {
+  if (a.rt) {
+    const int span = ((a.K + n_wg - 1) / n_wg + 7) & ~7;
+    const int k_beg = wg * span, k_end = min(a.K, k_beg + span);
+    for (int i = threadIdx.x; i < (k_end - k_beg) * a.r; i += blockDim.x) {
+      const int k = k_beg + i / a.r, c = i % a.r;
+      if constexpr (W32)
+        a.rt[(int64_t)k * a.r + c] = (_Float16)a.R32[(int64_t)c * a.K + k];
+      else
+        a.rt[(int64_t)k * a.r + c] = a.R[(int64_t)c * a.K + k];
+    }
+  }
+  if (a.bt || (W32 && a.b16)) {
+    const int span = ((a.N + n_wg - 1) / n_wg + 7) & ~7;
+    const int n_beg = wg * span, n_end = min(a.N, n_beg + span);
+    for (int i = threadIdx.x; i < (n_end - n_beg) * a.r; i += blockDim.x) {
+      const int n = n_beg + i / a.r, c = i % a.r;
+      const int64_t src = (int64_t)n * a.r + c;
+      _Float16 v;
+      if constexpr (W32) {
+        v = (_Float16)a.B32[src];
+        if (a.b16) a.b16[src] = v;
+      } else {
+        v = a.B[src];
+      }
+      if (a.bt) a.bt[(int64_t)c * a.N + n] = v;
+    }
+  }
 }
 
 // out[m][c] = fp16(s * sum_k drop(P)[m][k] * R[c][k]) for the 16*TB rows of row block rb, over
@@ -190,34 +224,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs& a, int rb, int slice,
       for (int v = 0; v < 4; v++)
         red[(wave * 16 * TB + 16 * t + 4 * g + v) * ld + 16 * b + (lane & 15)] = acc[t][b][v];
   }
-  // side outputs, spread over the workgroups: R^T [K, r], B^T [r, N] and (W32) fp16 B [N, r]
-  if (a.rt) {
-    const int span = ((a.K + n_wg - 1) / n_wg + 7) & ~7;
-    const int k_beg = wg * span, k_end = min(a.K, k_beg + span);
-    for (int i = threadIdx.x; i < (k_end - k_beg) * a.r; i += blockDim.x) {
-      const int k = k_beg + i / a.r, c = i % a.r;
-      if constexpr (W32)
-        a.rt[(int64_t)k * a.r + c] = (_Float16)a.R32[(int64_t)c * a.K + k];
-      else
-        a.rt[(int64_t)k * a.r + c] = a.R[(int64_t)c * a.K + k];
-    }
-  }
-  if (a.bt || (W32 && a.b16)) {
-    const int span = ((a.N + n_wg - 1) / n_wg + 7) & ~7;
-    const int n_beg = wg * span, n_end = min(a.N, n_beg + span);
-    for (int i = threadIdx.x; i < (n_end - n_beg) * a.r; i += blockDim.x) {
-      const int n = n_beg + i / a.r, c = i % a.r;
-      const int64_t src = (int64_t)n * a.r + c;
-      _Float16 v;
-      if constexpr (W32) {
-        v = (_Float16)a.B32[src];
-        if (a.b16) a.b16[src] = v;
-      } else {
-        v = a.B[src];
-      }
-      if (a.bt) a.bt[(int64_t)c * a.N + n] = v;
-    }
-  }
+  rows_side<W32>(a, wg, n_wg);
   __syncthreads();
   for (int i = threadIdx.x; i < 16 * TB * a.r; i += blockDim.x) {
     // consecutive threads: consecutive m of one outT row
@@ -240,11 +247,13 @@ template <int TB, int RB, bool R2>
 __global__ __launch_bounds__(1024) void k_lora_rows(RowsArgs a) {
   extern __shared__ float red[];  // [waves][16 * TB][r + 1]
   const int wg = (int)(blockIdx.y * gridDim.x + blockIdx.x), n_wg = (int)(gridDim.x * gridDim.y);
-  if (a.mask)
-    rows_block<false, TB, RB, true, R2>(a, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y,
+  if ((int)blockIdx.y >= a.slices)  // side outputs only
+    rows_side<false>(a, wg, n_wg);
+  else if (a.mask)
+    rows_block<false, TB, RB, true, R2>(a, (int)blockIdx.x, (int)blockIdx.y, a.slices,
                                         (int)blockDim.x >> 6, wg, n_wg, red);
   else
-    rows_block<false, TB, RB, false, false>(a, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y,
+    rows_block<false, TB, RB, false, false>(a, (int)blockIdx.x, (int)blockIdx.y, a.slices,
                                             (int)blockDim.x >> 6, wg, n_wg, red);
 }
 
@@ -266,7 +275,9 @@ __global__ __launch_bounds__(1024) void k_lora_rows_group(RowsGroup g) {
   int i = 0;
   while (i + 1 < g.n && bid >= g.start[i + 1]) i++;
   const int local = bid - g.start[i];
-  if (g.p[i].mask)
+  if (local >= g.rbs[i] * g.slices[i])  // side outputs only
+    rows_side<W32>(g.p[i], local, g.start[i + 1] - g.start[i]);
+  else if (g.p[i].mask)
     rows_block<W32, TB, RB, true, R2>(g.p[i], local % g.rbs[i], local / g.rbs[i], g.slices[i],
                                   g.nw[i], local, g.start[i + 1] - g.start[i], red);
   else
@@ -424,6 +435,17 @@ static int rows_tb(int r, int64_t workgroups_at_two, int64_t waves_at_two) {
   return r == 16 && workgroups_at_two >= 256 && waves_at_two >= 16 * 256 ? 2 : 1;
 }
 
+// Workgroups a rows problem gets past its row blocks, for its side outputs alone: with few tokens
+// the row blocks are few (one, times 4 slices, up to 16 tokens), and lora_A^T / lora_B^T written
+// by them alone took 40 us of a 56 us launch (gate and up at 4 tokens).  Enough that a thread
+// writes about four elements; none at 1024 tokens, whose row blocks are as many.
+static int64_t rows_extra(const RowsArgs& a, int64_t workgroups, int nw) {
+  const int64_t side = (a.rt ? (int64_t)a.K * a.r : 0) +
+                       (a.bt || a.b16 ? (int64_t)a.N * a.r : 0);
+  const int64_t want = side / (4 * 64 * nw);
+  return want > workgroups ? (want < 256 ? want : 256) - workgroups : 0;
+}
+
 // The row-product kernel with the dropout rounding the launch needs: twice (R2) where some
 // problem has a keep mask and rounding once is not the same for its scale.
 static bool rows_round2(const RowsArgs& a) { return a.mask && !round_once_exact(a.mscale); }
@@ -453,7 +475,11 @@ static int rows_launch(RowsArgs a, void* workspace, hipStream_t stream) {
   const int64_t at_two = (int64_t)((a.ldt + 31) / 32) * slices;
   const int tb = rows_tb(a.r, at_two, at_two * nw);
   const size_t lds = (size_t)nw * 16 * tb * (a.r + 1) * sizeof(float);
-  const dim3 grid((a.ldt + 16 * tb - 1) / (16 * tb), slices);
+  const int rbs = (a.ldt + 16 * tb - 1) / (16 * tb);
+  a.slices = slices;
+  int64_t extra = rows_extra(a, (int64_t)rbs * slices, nw);
+  extra = extra > 0 ? (extra + rbs - 1) / rbs : 0;
+  const dim3 grid(rbs, (unsigned)(slices + extra));
   const bool r2 = rows_round2(a);
   if (a.r != 16)
     launch_rows_k<1, kMaxRB>(r2, grid, dim3(64 * nw), lds, stream, a);
@@ -490,7 +516,9 @@ static int rows_group_launch(const RowsArgs* probs, int n, hipStream_t stream, b
   for (int i = 0; i < n; i++) {
     g.rbs[i] = (g.p[i].ldt + 16 * tb - 1) / (16 * tb);
     g.start[i] = total;
-    total += g.rbs[i] * g.slices[i];
+    const int wgs = g.rbs[i] * g.slices[i];
+    const int64_t extra = rows_extra(g.p[i], wgs, nw_max);
+    total += wgs + (extra > 0 ? (int)extra : 0);
   }
   g.start[n] = total;
   const size_t lds = (size_t)nw_max * 16 * tb * (r + 1) * sizeof(float);
