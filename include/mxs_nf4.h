@@ -127,7 +127,9 @@ int mxs_nf4_linear_fwd(const void* x, int M, int K, int N, const void* packed,
  * capture begins; the calls after it launch kernels only and are capturable.  A plan needing
  * more (splits * M * N * 4 bytes) returns MXS_ERR_SIZE with nothing launched.  Every call on
  * one GPU shares that array: calls that overlap in time on one GPU (other streams or threads)
- * race and must be serialized by the caller.  Same results as mxs_nf4_linear_fwd. */
+ * race and must be serialized by the caller.  Same results as mxs_nf4_linear_fwd, with the bits
+ * of its fused kernels (where its own plan decodes the weight into the workspace, at many tokens,
+ * and splits the reduction, the fp32 sums are added in another order). */
 int mxs_nf4_linear_fwd_noalloc(const void* x, int M, int K, int N, const void* packed,
                                const void* absmax8, const float* code, const float* absmax2,
                                const float* offset, const void* bias, const void* lora_h,

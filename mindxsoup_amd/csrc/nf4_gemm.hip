@@ -2153,6 +2153,7 @@ __global__ __launch_bounds__(64 * (4 + PW)) void k_nf4_gemm_ws_group(GemmGroup g
 }  // namespace mxs
 
 #include "dense_tile.h"
+#include "skinny.h"
 
 namespace mxs {
 
@@ -2267,8 +2268,37 @@ static int cu_count() {
   return counts[dev] > 0 ? counts[dev] : 0;
 }
 
-// Tile and split choice for one GEMM (M x Nc output, Kr reduction), from measured sweeps on
-// MI355X at the Qwen2.5-1.5B projection shapes (M = 1024):
+// The plans below are functions of sizes and the CU count that take up to some microseconds to
+// evaluate (a quarter of a whole small call's host time), so each thread keeps the last ones: a
+// direct-mapped table, an entry replaced by the next plan that falls on it.
+struct PlanKey {
+  int v[8];  // kind, CUs, sizes
+};
+
+template <class F>
+static std::array<int64_t, 3> plan_memo(const PlanKey& k, F&& make) {
+  struct Entry {
+    PlanKey key;
+    std::array<int64_t, 3> val;
+  };
+  thread_local Entry table[128];  // zero: kind 0 is no plan
+  uint32_t h = 2166136261u;
+  for (int x : k.v) h = (h ^ (uint32_t)x) * 16777619u;
+  Entry& e = table[(h ^ (h >> 15)) & 127];
+  if (!std::equal(k.v, k.v + 8, e.key.v)) {
+    e.val = make();
+    e.key = k;
+  }
+  return e.val;
+}
+
+enum PlanKind {
+  kPlanFew = 1, kPlanDense, kPlanPairSplits, kPlanDensePair, kPlanDenseSum, kPlanDenseGroup,
+  kPlanBytes
+};
+
+// Tile and split choice for one GEMM (M x Nc output, Kr reduction) at many tokens, from measured
+// sweeps on MI355X at the Qwen2.5-1.5B projection shapes (M = 1024):
 //   wide outputs (Nc >= 4096): warp-specialized 256x160, one tile per CU, no split;
 //   narrow outputs with a long reduction (Kr >= 4096): warp-specialized 256x96, split-K 4, with
 //   4 producer waves forward (46 against 51 us for down_proj at 1024 tokens) and 8 in the
@@ -2280,7 +2310,7 @@ static int cu_count() {
 //   (1430 tokens: 288 tiles of 128x64 would take two rounds, 25.6 against 19.2 us);
 //   small outputs: 64x128 all-wave tiles, split-K 4 when the reduction is long enough.
 // Splits keep at least 6 K-steps each.
-static void choose(int M, int Nc, int Kr, bool bwd, int* cfg, int* splits) {
+static void choose_base(int M, int Nc, int Kr, bool bwd, int* cfg, int* splits) {
   const int n_steps = Kr / kBK;
   int c, sp;
   if (Nc >= 4096) {
@@ -2298,6 +2328,67 @@ static void choose(int M, int Nc, int Kr, bool bwd, int* cfg, int* splits) {
   while (sp > 1 && n_steps / sp < 6) sp >>= 1;
   *cfg = c;
   *splits = sp;
+}
+
+static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Tiles of the warp-specialized configurations 6..12.
+static const int kWsBM[] = {256, 256, 128, 256, 128, 256, 128};
+static const int kWsBN[] = {128, 160, 128, 96, 128, 96, 64};
+
+// Time of one tile of `steps` K-steps with few CUs busy, in microseconds (HIP graphs; 24, 64, 140
+// and 172 steps of unsplit launches at 17 to 256 tokens, within 5 %).
+static double few_tile_us(int cfg, int steps) {
+  switch (cfg) {
+    case 12: return 0.33 * steps + 4.6;  // 128x64
+    case 10: return 0.52 * steps + 5.5;  // 128x128
+    case 9: return 0.52 * steps + 5.7;   // 256x96, forward
+    case 11: return 0.56 * steps + 9.0;  // 256x96, backward
+    case 6: return 0.63 * steps + 5.5;   // 256x128
+    default: return 0.79 * steps + 6.3;  // 256x160
+  }
+}
+
+static double few_us(int cus, int cfg, int sp, int M, int Nc, int steps) {
+  const int64_t wgs = ceil_div(M, kWsBM[cfg - 6]) * ceil_div(Nc, kWsBN[cfg - 6]) * sp;
+  const double t = ceil_div(wgs, cus) * few_tile_us(cfg, (int)ceil_div(steps, sp));
+  return sp > 1 ? t + 3.0 + (4.0 * sp + 2.0) * M * Nc / 5e6 : t;
+}
+
+// The planned configuration.  At up to 768 tokens the shapes' plans above leave most CUs idle (one
+// or two row bands: gate_proj 56 tiles of 256x160 at 256 tokens, down_proj 64 workgroups), and the
+// tile and split with the smallest estimate are taken where it is 8 % below the base plan's.
+// Measured, planned / base: gate forward 12.8 / 24.9 us at 64 tokens, 18.6 / 25.4 at 200, 20.1 /
+// 26.1 at 300, 28.1 / 32.8 at 700; down forward 15.0 / 27.4, 20.5 / 31.7, 24.8 / 33.0; a
+// 4096 x 11008 projection (wide and long: one split in the base plan) 24.6 / 57.3, 36.8 / 62.6,
+// 54.1 / 76.9.  A wide output's 24-step reduction stays whole, so that gate's and up's launches
+// of any kind keep one order of sums, and so does every short reduction of the input gradient.
+static void choose(int M, int Nc, int Kr, bool bwd, int* cfg, int* splits) {
+  choose_base(M, Nc, Kr, bwd, cfg, splits);
+  const int cus = cu_count();
+  if (M > 768 || Nc < 1024 || cus <= 0 || *cfg < 6) return;
+  const int base_cfg = *cfg, base_sp = *splits, steps = Kr / kBK;
+  const auto plan = plan_memo({{kPlanFew, cus, M, Nc, Kr, bwd}}, [&]() -> std::array<int64_t, 3> {
+    int best_c = base_cfg, best_sp = base_sp;
+    double best = 0.92 * few_us(cus, base_cfg, base_sp, M, Nc, steps);
+    for (int c : {12, 10, bwd ? 11 : 9, 6, 7})
+      for (int sp = 1; sp <= 8; sp++) {
+        if (sp > 1 &&
+            (steps / sp < 6 || !(Kr >= 4096 || (!bwd && Nc < 4096)) ||
+             (sp > base_sp && (int64_t)sp * M * Nc * 4 > (int64_t)MXS_NF4_SCRATCH_BYTES)))
+          break;
+        if (ceil_div(steps, ceil_div(steps, sp)) != sp) continue;
+        const double t = few_us(cus, c, sp, M, Nc, steps);
+        if (t < best) {
+          best = t;
+          best_c = c;
+          best_sp = sp;
+        }
+      }
+    return {best_c, best_sp, 0};
+  });
+  *cfg = (int)plan[0];
+  *splits = (int)plan[1];
 }
 
 // Argument checks of one GEMM problem: MXS_OK, an MXS_ERR_* code, or 1 when there is nothing
@@ -2352,6 +2443,7 @@ struct DensePlan {
 // against 66, not taken at 4096 (39 against 39).
 static double fused_tile_us(int cfg, int steps) {
   switch (cfg) {
+    case 6: return 0.95 * steps + 7.0;             // 256x128
     case 7: return 1.15 * steps + 8.0;             // 256x160
     case 9: case 11: return 0.87 * steps + 8.0;    // 256x96
     case 10: return 0.60 * steps + 6.5;            // 128x128
@@ -2368,17 +2460,13 @@ static double reduce_us(int splits, int M, int Nc) {
   return splits > 1 ? (4.0 * splits + 2.0) * M * Nc / 5.4e6 + 2.0 : 0.0;
 }
 
-static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
 // One GEMM on its fused plan (choose), or a negative number where the dense route is no
 // alternative (outputs narrower than 1024).
 static double fused_us(int M, int Nc, int Kr, bool bwd, bool glu) {
   int cfg, sp;
   choose(M, Nc, Kr, bwd, &cfg, &sp);
   if (cfg < 6) return -1.0;
-  static const int kBM[] = {256, 256, 128, 256, 128, 256, 128};  // cfg 6..12
-  static const int kBN[] = {128, 160, 128, 96, 128, 96, 64};
-  const int64_t tiles = ceil_div(M, kBM[cfg - 6]) * ceil_div(Nc, kBN[cfg - 6]) * sp;
+  const int64_t tiles = ceil_div(M, kWsBM[cfg - 6]) * ceil_div(Nc, kWsBN[cfg - 6]) * sp;
   const double tail = glu ? 11.3 : 0.0;  // the SwiGLU's gate / up traffic, per round
   return ceil_div(tiles, cu_count()) *
              (fused_tile_us(cfg, (int)ceil_div(Kr / kBK, sp)) + tail) +
@@ -2415,11 +2503,32 @@ static double dense_us(int M, int n, const int* Nc, int steps, int64_t values, b
   return best;
 }
 
+// `make` (which fills a plan and says whether the dense route is taken) through the memo.
+template <class F>
+static bool dense_memo(const PlanKey& k, DensePlan* d, F&& make) {
+  const auto v = plan_memo(k, [&]() -> std::array<int64_t, 3> {
+    DensePlan p{0, 0};
+    const bool ok = make(&p);
+    return {ok, p.bn, p.splits};
+  });
+  d->bn = (int)v[1];
+  d->splits = (int)v[2];
+  return v[0] != 0;
+}
+
+// Fewest tokens the dense route is considered at (its decode alone outweighs the row bands it
+// saves below).
+constexpr int kDenseTokens = 769;
+
 static bool dense_plan(int M, int Nc, int Kr, bool bwd, bool glu, DensePlan* d) {
-  const double f = fused_us(M, Nc, Kr, bwd, glu);
-  if (f < 0) return false;
-  const double t = dense_us(M, 1, &Nc, Kr / kBK, (int64_t)Nc * Kr, false, glu, 0, d);
-  return t > 0 && t < 0.95 * f;
+  const int cus = cu_count();
+  if (M < kDenseTokens || cus <= 0) return false;
+  return dense_memo({{kPlanDense, cus, M, Nc, Kr, bwd, glu}}, d, [&](DensePlan* p) {
+    const double f = fused_us(M, Nc, Kr, bwd, glu);
+    if (f < 0) return false;
+    const double t = dense_us(M, 1, &Nc, Kr / kBK, (int64_t)Nc * Kr, false, glu, 0, p);
+    return t > 0 && t < 0.95 * f;
+  });
 }
 
 // The copies' 32-bit offsets (a tile's rows of either operand) and whole keep words per tile.
@@ -2530,10 +2639,24 @@ static int launch_dense(bool bwd, const GemmArgs* probs, int n, bool sum, const 
   return splits > 1 && reduce ? launch_reduce(g.p[0], splits, stream) : MXS_OK;
 }
 
+// The few-token forward kernel takes up to 16 rows: a 1536 x 1536 projection at 1 token 4.2 us
+// against 11.3 on 128x64 tiles, 8960 x 1536 7.5 against 11.8 (and 27.9 on the 256x160 tiles the
+// wide shapes planned), 1536 x 8960 10.2 against 24.7; at 16 tokens 5.2, 9.7 and 14.0.  With a
+// second row block (17 to 32 rows) its operands spill: 25 us against 11.9 on 128x64 tiles
+// (8960 x 1536).
+static bool skinny_takes(int M, int Nc, int Kr) {
+  return M >= 1 && M <= kSkinnyRows && Nc > 0 && Kr > 0 && Kr % kBK == 0;
+}
+
 static int gemm_entry(bool bwd, const GemmArgs& a, int cfg, int splits, hipStream_t stream) {
   const int c = check_gemm(bwd, a);
   if (c != MXS_OK) return c == 1 ? MXS_OK : c;
   if (cfg < 0) {
+    if (!bwd && skinny_takes(a.M, a.Nc, a.Kr)) {
+      const int rc = launch_skinny(&a, 1, stream);
+      if (rc != MXS_OK || a.glu != 1) return rc;
+      return mxs_silu_mul(a.glu_g, a.C, a.glu_h, (int64_t)a.M * a.Nc, stream);
+    }
     DensePlan d;
     if (a.ws && (uintptr_t)a.ws % 16 == 0 && a.glu != 1 && a.cols_blocks == 0 &&
         dense_takes(a.M, a.Nc, a.Kr) && dense_plan(a.M, a.Nc, a.Kr, bwd, a.glu == 2, &d))
@@ -2557,12 +2680,10 @@ static bool grads_fusable(int M, int N, int K, int r, int* cfg_out, int* nw_out)
   if (cols_cpl(K + N) != kFusedColsCPL) return false;
   const int nw = cols_waves(M, r, kFusedColsCPL, cols_max_waves<kFusedColsCPL>());
   int cfg, sp;
-  choose(M, K, N, true, &cfg, &sp);
+  choose_base(M, K, N, true, &cfg, &sp);
   if (cfg < 6 || cfg >= kNumCfg || sp != 1) return false;
-  static const int kBM[] = {256, 256, 128, 256, 128, 256, 128};  // cfg 6..12
-  static const int kBN[] = {128, 160, 128, 96, 128, 96, 64};
   static const int kPW[] = {4, 4, 4, 4, 8, 8, 8};
-  const int bm = kBM[cfg - 6], bn = kBN[cfg - 6], pw = kPW[cfg - 6];
+  const int bm = kWsBM[cfg - 6], bn = kWsBN[cfg - 6], pw = kPW[cfg - 6];
   if (bm != 128) return false;  // only those kernels carry the gradient rows
   if (nw > 4 + pw) return false;
   if ((int64_t)K * N >= (int64_t(1) << 32) || (int64_t)bm * N * 2 >= (int64_t(1) << 32) ||
@@ -2598,9 +2719,8 @@ static bool glu_plan_ok(int M, int Nc, int Kr, bool bwd) {
   int cfg, sp;
   choose(M, Nc, Kr, bwd, &cfg, &sp);
   if (cfg < 6 || cfg >= kNumCfg) return false;
-  static const int kBM[] = {256, 256, 128, 256, 128, 256, 128};  // cfg 6..12
   static const int kPW[] = {4, 4, 4, 4, 8, 8, 8};
-  const int bm = kBM[cfg - 6], pw = kPW[cfg - 6];
+  const int bm = kWsBM[cfg - 6], pw = kPW[cfg - 6];
   return (int64_t)Nc * Kr < (int64_t(1) << 32) && (int64_t)bm * Kr * 2 < (int64_t(1) << 32) &&
          !(bwd && Nc < (pw == 8 ? 16 : 32));
 }
@@ -2940,25 +3060,53 @@ static int launch_ws_fwd_pair_mixed(const GemmArgs& a0, const GemmArgs& a1, int 
 static bool fwd_pair_plan_ok(int M, int N0, int N1, int K) {
   if (M <= 0 || N0 != N1 || K <= 0 || K % kBK) return false;
   int c, sp;
-  choose(M, N0, K, false, &c, &sp);
+  choose_base(M, N0, K, false, &c, &sp);
   return c == 7 && sp == 1 && (int64_t)N0 * K < (int64_t(1) << 32) &&
          (int64_t)256 * K * 2 < (int64_t(1) << 32);
 }
 
-// The pair's plan: both problems must plan the 256x96 split backward kernel (cfg 11) on their
-// own; the pair then splits each reduction kPairSplits ways.
-constexpr int kPairSplits = 2;
+// Splits of each of the pair's reductions (256x96 tiles, two problems): two, so that a workgroup
+// runs long (fixed costs paid half as often), or up to 8 where one or two row bands would leave
+// CUs idle (graph-timed with the reduce: 29.9 against 57.3 us at 64 tokens, 42.8 against 60.0 at
+// 300, 46.8 against 60.9 at 512).
+static int pair_splits(int M, const int N[2], int K) {
+  const int cus = cu_count();
+  if (cus <= 0 || M > 768) return 2;
+  const PlanKey key{{kPlanPairSplits, cus, M, K, N[0], N[1]}};
+  return (int)plan_memo(key, [&]() -> std::array<int64_t, 3> {
+    const int steps = std::max(N[0], N[1]) / kBK;
+    const int64_t tiles = ceil_div(M, 256) * ceil_div(K, 96) * 2;
+    int best = 2;
+    double bt = 0.0;
+    for (int sp = 2; sp <= 8; sp++) {
+      bool whole = true;  // every split of both problems has steps, and at least 6
+      for (int i = 0; i < 2; i++) {
+        const int st = N[i] / kBK;
+        whole = whole && st / sp >= 6 && ceil_div(st, ceil_div(st, sp)) == sp;
+      }
+      if (!whole && sp > 2) continue;
+      const double t = ceil_div(tiles * sp, cus) * few_tile_us(11, (int)ceil_div(steps, sp)) +
+                       (8.0 * sp + 2.0) * M * K / 5e6;
+      if (sp == 2 || t < 0.92 * bt) {
+        bt = t;
+        best = sp;
+      }
+    }
+    return {best, 0, 0};
+  })[0];
+}
 
+// The pair's plan: both problems' base plan is the 256x96 split backward kernel (cfg 11).
 static bool pair_plan_ok(int M, int N0, int N1, int K) {
   if (M <= 0 || K <= 0 || N0 <= 0 || N1 <= 0 || N0 % kBK || N1 % kBK || K % kBK) return false;
   for (int n : {N0, N1}) {
     int cfg, sp;
-    choose(M, K, n, true, &cfg, &sp);
+    choose_base(M, K, n, true, &cfg, &sp);
     if (cfg != 11 || sp == 1) return false;
     if ((int64_t)K * n >= (int64_t(1) << 32) || (int64_t)256 * n * 2 >= (int64_t(1) << 32))
       return false;
-    const int steps = n / kBK, sps = (steps + kPairSplits - 1) / kPairSplits;
-    if (steps < kPairSplits || (steps + sps - 1) / sps != kPairSplits) return false;
+    const int steps = n / kBK, sps = (steps + 1) / 2;
+    if (steps < 2 || (steps + sps - 1) / sps != 2) return false;
   }
   return true;
 }
@@ -2986,29 +3134,38 @@ static int64_t dense_sum_bytes(int n, int M, const int* N, int K, const DensePla
 // tokens: 469 us and 19 us of decode against 613 us and a reduce of four planes; at 3001 tokens
 // 192 + 17 (and a reduce of two planes instead of four) against 212.
 static bool dense_pair_plan(int M, const int N[2], int K, DensePlan* d) {
-  if (cu_count() <= 0 || !dense_takes_all(2, M, N, K, true)) return false;
-  int steps = 0, longest = 0;
-  for (int i = 0; i < 2; i++) {
-    steps += N[i] / kBK;
-    longest = std::max(longest, N[i] / kBK);
-  }
-  const double f = ceil_div(ceil_div(M, 256) * ceil_div(K, 96) * 2 * kPairSplits, cu_count()) *
-                       fused_tile_us(11, (int)ceil_div(longest, kPairSplits)) +
-                   reduce_us(2 * kPairSplits, M, K);
-  const double t = dense_us(M, 2, &K, steps, weight_values(2, N, K), true, false, 0, d);
-  return t > 0 && t < 0.95 * f;
+  const int cus = cu_count();
+  if (cus <= 0 || M < kDenseTokens || !dense_takes_all(2, M, N, K, true)) return false;
+  return dense_memo({{kPlanDensePair, cus, M, K, N[0], N[1]}}, d, [&](DensePlan* p) {
+    int steps = 0, longest = 0;
+    for (int i = 0; i < 2; i++) {
+      steps += N[i] / kBK;
+      longest = std::max(longest, N[i] / kBK);
+    }
+    const int sp = pair_splits(M, N, K);
+    const double f = ceil_div(ceil_div(M, 256) * ceil_div(K, 96) * 2 * sp, cus) *
+                         fused_tile_us(11, (int)ceil_div(longest, sp)) +
+                     reduce_us(2 * sp, M, K);
+    const double t = dense_us(M, 2, &K, steps, weight_values(2, N, K), true, false, 0, p);
+    return t > 0 && t < 0.95 * f;
+  });
 }
 
 // q, k and v's summed dX without their gradients (against one launch of 128x128 tiles): 84 us
 // and 5 us of decode against 110 at 8192 tokens.
 static bool dense_sum_plan(int n, int M, const int* N, int K, DensePlan* d) {
-  if (cu_count() <= 0 || n < 2 || n > kMaxSum || !dense_takes_all(n, M, N, K, true)) return false;
-  int steps = 0;
-  for (int i = 0; i < n; i++) steps += N[i] / kBK;
-  const double f = ceil_div(ceil_div(M, 128) * ceil_div(K, 128), cu_count()) *
-                   (fused_tile_us(10, steps) + 8.0);
-  const double t = dense_us(M, n, &K, steps, weight_values(n, N, K), true, false, 0, d);
-  return t > 0 && t < 0.95 * f;
+  const int cus = cu_count();
+  if (cus <= 0 || M < kDenseTokens || n < 2 || n > kMaxSum || !dense_takes_all(n, M, N, K, true))
+    return false;
+  const PlanKey key{{kPlanDenseSum, cus, M, K, N[0], N[1], n > 2 ? N[2] : 0}};
+  return dense_memo(key, d, [&](DensePlan* p) {
+    int steps = 0;
+    for (int i = 0; i < n; i++) steps += N[i] / kBK;
+    const double f = ceil_div(ceil_div(M, 128) * ceil_div(K, 128), cus) *
+                     (fused_tile_us(10, steps) + 8.0);
+    const double t = dense_us(M, n, &K, steps, weight_values(n, N, K), true, false, 0, p);
+    return t > 0 && t < 0.95 * f;
+  });
 }
 
 // Several forwards over one input in one launch: q, k and v (against 128x128 tiles; 70 us, rotated,
@@ -3016,22 +3173,28 @@ static bool dense_sum_plan(int n, int M, const int* N, int K, DensePlan* d) {
 // tiles of which a mixed launch saves 5 %; 448 + 15 against 527 us at 8192, 164 + 14 against 209
 // at 3001).
 static bool dense_group_plan(int n, int M, const int* N, int K, bool rope, DensePlan* d) {
-  if (cu_count() <= 0 || n < 1 || n > kMaxGemmGroup || !dense_takes_all(n, M, N, K, false))
+  const int cus = cu_count();
+  if (cus <= 0 || M < kDenseTokens || n < 1 || n > kMaxGemmGroup ||
+      !dense_takes_all(n, M, N, K, false))
     return false;
-  bool wide = true;
-  int64_t tiles128 = 0, tiles160 = 0;
-  for (int i = 0; i < n; i++) {
-    wide = wide && N[i] >= 4096;
-    tiles128 += ceil_div(M, 128) * ceil_div(N[i], 128);
-    tiles160 += ceil_div(M, 256) * ceil_div(N[i], 160);
-  }
-  const int steps = K / kBK;
-  const double f = wide && !rope
-      ? 0.95 * ceil_div(tiles160, cu_count()) * fused_tile_us(7, steps)
-      : ceil_div(tiles128, cu_count()) * (fused_tile_us(10, steps) + (rope ? 5.5 : 0.0));
-  const double t = dense_us(M, n, N, steps, weight_values(n, N, K), false, false, rope ? 256 : 0,
-                            d);
-  return t > 0 && t < 0.95 * f;
+  PlanKey key{{kPlanDenseGroup + 16 * rope, cus, M, K}};
+  for (int i = 0; i < n; i++) key.v[4 + i] = N[i];
+  return dense_memo(key, d, [&](DensePlan* p) {
+    bool wide = true;
+    int64_t tiles128 = 0, tiles160 = 0;
+    for (int i = 0; i < n; i++) {
+      wide = wide && N[i] >= 4096;
+      tiles128 += ceil_div(M, 128) * ceil_div(N[i], 128);
+      tiles160 += ceil_div(M, 256) * ceil_div(N[i], 160);
+    }
+    const int steps = K / kBK;
+    const double f = wide && !rope
+        ? 0.95 * ceil_div(tiles160, cus) * fused_tile_us(7, steps)
+        : ceil_div(tiles128, cus) * (fused_tile_us(10, steps) + (rope ? 5.5 : 0.0));
+    const double t = dense_us(M, n, N, steps, weight_values(n, N, K), false, false, rope ? 256 : 0,
+                              p);
+    return t > 0 && t < 0.95 * f;
+  });
 }
 
 // The arguments of a dX GEMM whose launch also computes the LoRA gradients (its workgroups past
@@ -3111,7 +3274,7 @@ static bool dx_grads_sum_ok(int n, int M, const int* N, int K, int r, bool grads
     // N = 8960) re-reads dY from L2 for every column tile (154 against 101 us for the split-K
     // pair at 1024 tokens)
     int cfg, sp;
-    choose(M, K, N[i], true, &cfg, &sp);
+    choose_base(M, K, N[i], true, &cfg, &sp);
     if (sp != 1) return false;
     if (grads && cols_cpl(K + N[i]) != kFusedColsCPL) return false;
     if (grads) cols += (K + WC - 1) / WC + (N[i] + WC - 1) / WC;
@@ -3140,19 +3303,25 @@ using namespace mxs;
 
 // Split-K workspace: one fp32 partial plane per split.
 int64_t mxs_nf4_gemm_workspace_bytes(int M, int Nc, int Kr, int cfg, int splits) {
-  int64_t dense = 0;
-  if (cfg < 0) {
+  if (cfg >= 0)
+    return splits > 1 ? (int64_t)splits * M * Nc * (int64_t)sizeof(float) : 0;
+  const auto v = plan_memo({{kPlanBytes, cu_count(), M, Nc, Kr}}, [&]() -> std::array<int64_t, 3> {
+    int64_t need = 0;
+    int c, sp;
+    for (bool bwd : {false, true}) {  // a caller may use one workspace for both directions
+      choose(M, Nc, Kr, bwd, &c, &sp);
+      if (sp > 1) need = std::max(need, (int64_t)sp * M * Nc * (int64_t)sizeof(float));
+    }
     if (dense_takes(M, Nc, Kr))
-      for (int v = 0; v < 3; v++) {  // forward, backward, backward with the SwiGLU adjoint
+      for (int k = 0; k < 3; k++) {  // forward, backward, backward with the SwiGLU adjoint
         DensePlan d;
-        if (!dense_plan(M, Nc, Kr, v > 0, v > 1, &d)) continue;
+        if (!dense_plan(M, Nc, Kr, k > 0, k > 1, &d)) continue;
         const int64_t planes = d.splits > 1 ? (int64_t)d.splits * M * Nc * 4 : 0;
-        dense = std::max(dense, w16_bytes(Nc, Kr) + planes);
+        need = std::max(need, w16_bytes(Nc, Kr) + planes);
       }
-    choose(M, Nc, Kr, false, &cfg, &splits);  // both directions split alike
-  }
-  if (splits <= 1) return dense;
-  return std::max(dense, (int64_t)splits * M * Nc * (int64_t)sizeof(float));
+    return {need, 0, 0};
+  });
+  return v[0];
 }
 
 static void set_workspace(GemmArgs& a, void* workspace) {
@@ -3588,6 +3757,11 @@ int mxs_nf4_linear_fwd_hp_pair(const void* x, int M, int K, const int N[2],
     if (c != MXS_OK) return c == 1 ? MXS_OK : c;
     p[i] = a;
   }
+  if (skinny_takes(M, N[0], K)) return launch_skinny(p, 2, stream);
+  // 256x96 tiles where both projections' fit the CUs at once (up to 256 tokens at 8960 columns:
+  // 188 tiles, 24.6 us against 31.3 for 112 of 256x160; at 17 tokens 21.5 against 27.6)
+  if (2 * ceil_div(M, 256) * ceil_div(N[0], 96) <= cu_count())
+    return launch_ws_fwd_pair<256, 96, 4, 1, 4, 4>(p[0], p[1], stream);
   const int ncut = fwd_pair_mixed_cut(M, N[0], K);
   if (ncut > 0) return launch_ws_fwd_pair_mixed(p[0], p[1], ncut, stream);
   return launch_ws_fwd_pair<256, 160, 4, 1, 4, 4>(p[0], p[1], stream);
@@ -3599,8 +3773,8 @@ int mxs_nf4_linear_bwd_dx_pair_ok(int M, int N0, int N1, int K) {
 
 int64_t mxs_nf4_linear_bwd_dx_pair_workspace_bytes(int M, int N0, int N1, int K) {
   if (!pair_plan_ok(M, N0, N1, K)) return 0;
-  const int64_t fused = (int64_t)2 * kPairSplits * M * K * (int64_t)sizeof(float);
   const int N[2] = {N0, N1};
+  const int64_t fused = (int64_t)2 * pair_splits(M, N, K) * M * K * (int64_t)sizeof(float);
   DensePlan d;
   return dense_pair_plan(M, N, K, &d) ? std::max(fused, dense_sum_bytes(2, M, N, K, d)) : fused;
 }
@@ -3621,7 +3795,7 @@ int mxs_nf4_linear_bwd_dx_hp_pair(const void* const dy[2], int M, const int N[2]
   DensePlan d;
   if (dense_pair_plan(M, N, K, &d) && (uintptr_t)workspace % 16 == 0)
     return launch_dense(true, p, 2, true, d, workspace, true, nullptr, stream);
-  return launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], kPairSplits, stream);
+  return launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], pair_splits(M, N, K), stream);
 }
 
 int mxs_nf4_linear_bwd_dx_hp_pair_grads(
@@ -3655,7 +3829,8 @@ int mxs_nf4_linear_bwd_dx_hp_pair_grads(
     if (e != MXS_OK) return e;
     if (cols_cpl(K + N[i]) != cpl) return MXS_ERR_SIZE;
   }
-  int planes = 2 * kPairSplits;
+  const int sp = pair_splits(M, N, K);
+  int planes = 2 * sp;
   DensePlan d;
   if (dense_pair_plan(M, N, K, &d) && (uintptr_t)workspace % 16 == 0) {
     const int e = launch_dense(true, p, 2, true, d, workspace, false, &p[0].ws, stream);
@@ -3667,7 +3842,7 @@ int mxs_nf4_linear_bwd_dx_hp_pair_grads(
                                   da, db, stream);
   } else {
     const int e =
-        launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], kPairSplits, stream, false);
+        launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], sp, stream, false);
     if (e != MXS_OK) return e;
   }
   if (cpl == 8) return reduce_cols_launch<8>(p[0], planes, g, M, ldt, r, stream);
@@ -3744,6 +3919,7 @@ static int fwd_hp_group(int n, const void* const x[], int M, int K, const int N[
     probs[live++] = a;
   }
   if (live == 0) return MXS_OK;
+  if (rs.n_rope == 0 && skinny_takes(M, 1, K)) return launch_skinny(probs, live, stream);
   DensePlan d;
   if (workspace && live == n && dense_group_plan(n, M, N, K, rs.n_rope > 0, &d))
     return launch_dense(false, probs, n, false, d, workspace, true, nullptr, stream);
@@ -3899,6 +4075,9 @@ extern "C" int mxs_nf4_linear_fwd_noalloc(const void* x, int M, int K, int N, co
                                           const void* lora_b, int r, void* y, int cfg,
                                           int splits, hipStream_t stream) {
   if (M < 0 || K < 0 || N < 0) return MXS_ERR_ARG;
+  if (cfg < 0 && skinny_takes(M, N, K))
+    return mxs_nf4_linear_fwd(x, M, K, N, packed, absmax8, code, absmax2, offset, bias, lora_h,
+                              lora_b, r, y, nullptr, -1, 1, stream);
   if (cfg < 0) choose(M, N, K, false, &cfg, &splits);
   // the split count the launch will use (launch_cfg / launch_ws clamp it the same way)
   const int n_steps = K / kBK;
