@@ -16,6 +16,7 @@
 //   lora_bwd          its dX, dA, dB (solution/dropout.py:62-69 for the dropout's gradient)
 //   lora_fwd_group    lora_fwd for 1..4 projections reading one input (q/k/v; gate/up)
 //   lora_bwd_group    lora_bwd for them, small launches shared
+//   mlp_fwd, mlp_bwd  the SwiGLU MLP block of three such projections (solution/mlp.py:33-44)
 // Autograd ops (one node per call; backward in C++), named as the package's Python Functions
 // they stand for (a node's name() says which ran):
 //   linear         NF4LinearFunction
@@ -373,6 +374,8 @@ Tensor lora_w(const Tensor& t, int64_t rows, int64_t cols, const at::Device& dev
 // (mxs_nf4_linear_fwd_hp), which finish Hs and compute Y = x W^T + bias + Hs B^T and write
 // Hs^T.  Returns (ys, hts, ats, bts).  For one projection this is lora_fwd: the grouped rows
 // launch of one problem gives the bits of mxs_lora_h_partials.
+// side = false (no backward will follow): no lora_A^T, lora_B^T or Hs^T is written; hts, ats and
+// bts come back undefined.
 // The RoPE the grouped forward may fold into its first n_rope outputs (attention's q / k):
 // cos / sin fp32 [1 or B, T, 128], one layout, unit last stride; x's rows B sequences of T.
 struct RopeOperands {
@@ -413,7 +416,7 @@ Lists4 fwd_impl(const Tensor& x, TensorList lora_a, TensorList lora_b, TensorLis
                 TensorList absmax8, TensorList code, TensorList absmax2, TensorList offset,
                 const std::vector<OptTensor>& bias, const std::vector<OptTensor>& keep,
                 double mask_scale, double s, bool one_gemm, const OptTensor& cos = std::nullopt,
-                const OptTensor& sin = std::nullopt, int64_t n_rope = 0) {
+                const OptTensor& sin = std::nullopt, int64_t n_rope = 0, bool side = true) {
   const size_t n = lora_a.size();
   check_group(n, {lora_b.size(), packed.size(), absmax8.size(), code.size(), absmax2.size(),
                   offset.size(), bias.size(), keep.size()});
@@ -451,8 +454,10 @@ Lists4 fwd_impl(const Tensor& x, TensorList lora_a, TensorList lora_b, TensorLis
     masks[i] = keep_mask(keep[i], M, K, dev);
     biases[i] = bias16(bias[i], N, dev);
     hps[i] = at::empty({S, ldt, r}, f16.dtype(at::kFloat));
-    ats[i] = at::empty({K, r}, f16);
-    bts[i] = at::empty({r, N}, f16);
+    if (side) {
+      ats[i] = at::empty({K, r}, f16);
+      bts[i] = at::empty({r, N}, f16);
+    }
     Ns[i] = as_int(N, "N");
     Ks[i] = k;
     xs[i] = xc.data_ptr();
@@ -468,8 +473,8 @@ Lists4 fwd_impl(const Tensor& x, TensorList lora_a, TensorList lora_b, TensorLis
     p_off[i] = w[i].offset;
     p_hpw[i] = hps[i].data_ptr<float>();
     p_hp[i] = p_hpw[i];
-    p_at[i] = ats[i].data_ptr();
-    p_bt[i] = bts[i].data_ptr();
+    p_at[i] = ptr(ats[i]);
+    p_bt[i] = ptr(bts[i]);
     p_b16[i] = b16[i].data_ptr();
   }
   const RopeOperands rope = rope_operands(cos, sin, n_rope, M, n, dev);
@@ -494,9 +499,9 @@ Lists4 fwd_impl(const Tensor& x, TensorList lora_a, TensorList lora_b, TensorLis
   }
   for (size_t i = 0; i < n; ++i) {
     ys[i] = at::empty({M, Ns[i]}, f16);
-    hts[i] = at::empty({r, ldt}, f16);
+    if (side) hts[i] = at::empty({r, ldt}, f16);
     p_y[i] = ys[i].data_ptr();
-    p_ht[i] = hts[i].data_ptr();
+    p_ht[i] = ptr(hts[i]);
   }
   // many tokens: every weight decoded once into a workspace, then one fp16 GEMM launch
   const bool pair = !one_gemm && n == 2 && mxs_nf4_linear_fwd_pair_ok(m, Ns[0], Ns[1], k);
@@ -1091,6 +1096,158 @@ Lists3 lora_bwd_group_meta(TensorList dy, const Tensor& x, const OptTensorList&,
   return {dxs, das, dbs};
 }
 
+// ---- the MLP block -------------------------------------------------------------------------------
+
+// down(silu(gate(x)) * up(x)) for three NF4 + LoRA projections (gate, up, down in every list),
+// NF4LoraMLPFunction.forward's launches: gate's and up's row products and GEMMs shared, the
+// elementwise SwiGLU, down.  gate and up share one scaling and dropout rate (the caller checks).
+// Returns y, or for a backward (train) y, gate, up, h, then hts, ats, bts and the keep bits of
+// the three (undefined without dropout).
+std::vector<Tensor> mlp_fwd_cuda(const Tensor& x, TensorList lora_a, TensorList lora_b,
+                                 TensorList packed, TensorList absmax8, TensorList code,
+                                 TensorList absmax2, TensorList offset,
+                                 const OptTensorList& bias, const OptTensorList& keep,
+                                 at::ArrayRef<double> mask_scale, at::ArrayRef<double> s,
+                                 bool train) {
+  check_group(3, {lora_a.size(), lora_b.size(), packed.size(), absmax8.size(), code.size(),
+                  absmax2.size(), offset.size(), mask_scale.size(), s.size()});
+  TORCH_CHECK(s[0] == s[1] && mask_scale[0] == mask_scale[1],
+              "gate and up need one LoRA scaling and one dropout rate");
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2, "x must be fp16 [M, K] on the GPU");
+  const at::OptionalDeviceGuard guard(at::device_of(x));
+  const at::Device dev = x.device();
+  const auto kp = entries(keep, 3), bs = entries(bias, 3);
+  const int64_t inter = lora_b[0].size(0);
+  TORCH_CHECK(lora_b[1].size(0) == inter, "gate and up must have one width");
+  const auto gk = keep_masks({kp[0], kp[1]}, x.size(0), x.size(1), dev);
+  const Tensor dk = keep_mask(kp[2], x.size(0), inter, dev);
+  auto opt = [](const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); };
+  auto sl = [](TensorList l, size_t b, size_t n) { return l.slice(b, n); };
+  auto [ys, hts, ats, bts] =
+      fwd_impl(x, sl(lora_a, 0, 2), sl(lora_b, 0, 2), sl(packed, 0, 2), sl(absmax8, 0, 2),
+               sl(code, 0, 2), sl(absmax2, 0, 2), sl(offset, 0, 2), {bs[0], bs[1]},
+               {opt(gk[0]), opt(gk[1])}, mask_scale[0], s[0], false, std::nullopt, std::nullopt,
+               0, train);
+  Tensor h = at::empty_like(ys[0]);
+  ok(mxs_silu_mul(ys[0].data_ptr(), ys[1].data_ptr(), h.data_ptr(), h.numel(), stream_of(h)),
+     "mxs_silu_mul");
+  if (!train) ys.clear();  // gate and up are read no more
+  auto [yd, htd, atd, btd] =
+      fwd_impl(h, sl(lora_a, 2, 1), sl(lora_b, 2, 1), sl(packed, 2, 1), sl(absmax8, 2, 1),
+               sl(code, 2, 1), sl(absmax2, 2, 1), sl(offset, 2, 1), {bs[2]}, {opt(dk)},
+               mask_scale[2], s[2], false, std::nullopt, std::nullopt, 0, train);
+  if (!train) return {yd[0]};
+  return {yd[0], ys[0], ys[1], h, hts[0], hts[1], htd[0], ats[0], ats[1], atd[0],
+          bts[0], bts[1], btd[0], gk[0], gk[1], dk};
+}
+
+std::vector<Tensor> mlp_fwd_meta(const Tensor& x, TensorList lora_a, TensorList lora_b,
+                                 TensorList, TensorList, TensorList, TensorList, TensorList,
+                                 const OptTensorList&, const OptTensorList& keep,
+                                 at::ArrayRef<double>, at::ArrayRef<double>, bool train) {
+  const int64_t M = x.size(0), hidden = x.size(1), inter = lora_b[0].size(0);
+  const auto o = x.options().dtype(at::kHalf);
+  Tensor y = at::empty({M, lora_b[2].size(0)}, o);
+  if (!train) return {y};
+  std::vector<Tensor> out{y};
+  for (int i = 0; i < 3; ++i) out.push_back(at::empty({M, inter}, o));
+  for (int i = 0; i < 3; ++i) out.push_back(at::empty({lora_a[i].size(0), ldt_of(M)}, o));
+  for (int i = 0; i < 3; ++i) out.push_back(at::empty({lora_a[i].size(1), lora_a[i].size(0)}, o));
+  for (int i = 0; i < 3; ++i) out.push_back(at::empty({lora_b[i].size(1), lora_b[i].size(0)}, o));
+  for (int i = 0; i < 3; ++i) {
+    const OptTensor k = entry(keep, i);
+    out.push_back(k.has_value() && k->defined()
+                      ? at::empty({M, ((i < 2 ? hidden : inter) + 31) / 32}, o.dtype(at::kInt))
+                      : Tensor());
+  }
+  return out;
+}
+
+// Its backward (NF4LoraMLPFunction.backward): down's dX GEMM with the SwiGLU adjoint, which writes
+// d(gate) and d(up) over gate and up; down's dA / dB; up's and gate's backward with their launches
+// shared and their input gradients summed.  wants: x, then dA and dB of gate, up and down.
+// Returns dx and those six, undefined where not wanted.
+std::vector<Tensor> mlp_bwd_cuda(const Tensor& dy, const Tensor& x, const Tensor& gate,
+                                 const Tensor& up, const Tensor& h, const OptTensorList& keep,
+                                 TensorList ht, TensorList at_, TensorList bt, TensorList packed,
+                                 TensorList absmax8, TensorList code, TensorList absmax2,
+                                 TensorList offset, at::ArrayRef<double> mask_scale,
+                                 at::ArrayRef<double> s, at::IntArrayRef wants) {
+  check_group(3, {ht.size(), at_.size(), bt.size(), packed.size(), absmax8.size(), code.size(),
+                  absmax2.size(), offset.size(), mask_scale.size(), s.size()});
+  TORCH_CHECK(wants.size() == 7, "wants: x, then dA and dB of gate, up and down");
+  TORCH_CHECK(dy.is_cuda(), "dy must be on the GPU");
+  const at::OptionalDeviceGuard guard(at::device_of(dy));
+  const auto kp = entries(keep, 3);
+  const BwdOperands o = bwd_operands(dy, h, kp[2], ht[2], at_[2], bt[2], packed[2], absmax8[2],
+                                     code[2], absmax2[2], offset[2], dy.device());
+  TORCH_CHECK(gate.sizes() == h.sizes() && up.sizes() == h.sizes() &&
+                  gate.scalar_type() == at::kHalf && up.scalar_type() == at::kHalf &&
+                  gate.is_contiguous() && up.is_contiguous(),
+              "gate and up must be contiguous fp16 of h's shape");
+  const hipStream_t st = stream_of(o.dy);
+  const auto f16 = o.x.options();
+  const float ms = static_cast<float>(mask_scale[2]);
+  const bool wa = wants[5] != 0, wb = wants[6] != 0;
+  Tensor da, db;
+  {
+    Tensor dhp = at::empty({mxs_lora_slices(o.M, o.N), o.ldt, o.r}, f16.dtype(at::kFloat));
+    ok(mxs_lora_dh_partials(o.dy.data_ptr(), o.M, o.N, o.bt.data_ptr(), o.r,
+                            static_cast<float>(s[2]), o.ldt, dhp.data_ptr<float>(), st),
+       "mxs_lora_dh_partials");
+    Tensor dht = wa || wb ? at::empty({o.r, o.ldt}, f16) : Tensor();
+    const Tensor ws = gemm_ws_bwd(o);
+    if (mxs_nf4_linear_glu_fused(o.M, o.N, o.K, 1)) {
+      ok(mxs_nf4_linear_bwd_dx_glu(o.dy.data_ptr(), o.M, o.N, o.K, o.w.packed, o.w.absmax8,
+                                   o.w.code, o.w.absmax2, o.w.offset, dhp.data_ptr<float>(),
+                                   (int)dhp.size(0), o.ldt, o.at.data_ptr(), o.r, ptr(o.mask),
+                                   ms, ptr(dht), gate.data_ptr(), up.data_ptr(), ptr(ws), st),
+         "mxs_nf4_linear_bwd_dx_glu");
+    } else {
+      Tensor dh = at::empty_like(o.x);
+      ok(mxs_nf4_linear_bwd_dx_hp(o.dy.data_ptr(), o.M, o.N, o.K, o.w.packed, o.w.absmax8,
+                                  o.w.code, o.w.absmax2, o.w.offset, dhp.data_ptr<float>(),
+                                  (int)dhp.size(0), o.ldt, o.at.data_ptr(), o.r, ptr(o.mask), ms,
+                                  ptr(dht), dh.data_ptr(), ptr(ws), -1, 1, st),
+         "mxs_nf4_linear_bwd_dx_hp");
+      ok(mxs_silu_mul_bwd(dh.data_ptr(), gate.data_ptr(), up.data_ptr(), dh.numel(), st),
+         "mxs_silu_mul_bwd");
+    }
+    if (wa) da = at::empty({o.r, o.K}, f16.dtype(at::kFloat));
+    if (wb) db = at::empty({o.N, o.r}, f16.dtype(at::kFloat));
+    if (wa || wb)
+      ok(mxs_lora_grads(dht.data_ptr(), o.ht.data_ptr(), o.ldt, o.x.data_ptr(), o.dy.data_ptr(),
+                        o.M, o.K, o.N, o.r, ptr(o.mask), ms, ptr<float>(da), ptr<float>(db),
+                        nullptr, st),
+         "mxs_lora_grads");
+  }
+  // up, then gate (the order of solution/mlp_tail.py:42-46)
+  auto two = [](TensorList l) { return std::array<Tensor, 2>{l[1], l[0]}; };
+  OptTensorList k2;
+  k2.push_back(kp[1]);
+  k2.push_back(kp[0]);
+  const std::array<Tensor, 2> dys{up, gate};
+  const std::array<int64_t, 6> w2{wants[0], wants[3], wants[4], wants[0], wants[1], wants[2]};
+  auto [dxs, das, dbs] = lora_bwd_group_cuda(
+      dys, x, k2, two(ht), two(at_), two(bt), two(packed), two(absmax8), two(code), two(absmax2),
+      two(offset), mask_scale[0], s[0], w2, true);
+  return {dxs[0], das[1], dbs[1], das[0], dbs[0], da, db};
+}
+
+std::vector<Tensor> mlp_bwd_meta(const Tensor& dy, const Tensor& x, const Tensor&, const Tensor&,
+                                 const Tensor&, const OptTensorList&, TensorList, TensorList at_,
+                                 TensorList bt, TensorList, TensorList, TensorList, TensorList,
+                                 TensorList, at::ArrayRef<double>, at::ArrayRef<double>,
+                                 at::IntArrayRef wants) {
+  const auto f32 = x.options().dtype(at::kFloat);
+  std::vector<Tensor> out{wants[0] ? at::empty_like(x) : Tensor()};
+  for (int i = 0; i < 3; ++i) {
+    out.push_back(wants[1 + 2 * i] ? at::empty({at_[i].size(1), at_[i].size(0)}, f32) : Tensor());
+    out.push_back(wants[2 + 2 * i] ? at::empty({bt[i].size(1), bt[i].size(0)}, f32) : Tensor());
+  }
+  return out;
+}
+
 // ---- autograd ----------------------------------------------------------------------------------
 // The autograd ops reach the device ops through the dispatcher below the autograd keys, so that
 // a fake-tensor or meta call takes their Meta kernels.
@@ -1388,6 +1545,13 @@ TORCH_LIBRARY(mxs_nf4, m) {
         "Tensor[] bt, Tensor[] packed, Tensor[] absmax8, Tensor[] code, Tensor[] absmax2, "
         "Tensor[] offset, float mask_scale, float s, int[] wants, bool sum_dx=False) "
         "-> (Tensor[], Tensor[], Tensor[])");
+  m.def("mlp_fwd(Tensor x, Tensor[] lora_a, Tensor[] lora_b, Tensor[] packed, Tensor[] absmax8, "
+        "Tensor[] code, Tensor[] absmax2, Tensor[] offset, Tensor?[] bias, Tensor?[] keep, "
+        "float[] mask_scale, float[] s, bool train) -> Tensor[]");
+  m.def("mlp_bwd(Tensor dy, Tensor x, Tensor(a!) gate, Tensor(b!) up, Tensor h, Tensor?[] keep, "
+        "Tensor[] ht, Tensor[] at, Tensor[] bt, Tensor[] packed, Tensor[] absmax8, "
+        "Tensor[] code, Tensor[] absmax2, Tensor[] offset, float[] mask_scale, float[] s, "
+        "int[] wants) -> Tensor[]");
   m.def("linear(Tensor x, Tensor packed, Tensor absmax8, Tensor code, Tensor absmax2, "
         "Tensor offset, int out_features, Tensor? bias) -> Tensor");
   m.def("lora_linear(Tensor x, Tensor lora_a, Tensor lora_b, Tensor packed, Tensor absmax8, "
@@ -1407,6 +1571,8 @@ TORCH_LIBRARY_IMPL(mxs_nf4, CUDA, m) {
   m.impl("lora_bwd", &lora_bwd_cuda);
   m.impl("lora_fwd_group", &lora_fwd_group_cuda);
   m.impl("lora_bwd_group", &lora_bwd_group_cuda);
+  m.impl("mlp_fwd", &mlp_fwd_cuda);
+  m.impl("mlp_bwd", &mlp_bwd_cuda);
 }
 
 TORCH_LIBRARY_IMPL(mxs_nf4, Meta, m) {
@@ -1417,6 +1583,8 @@ TORCH_LIBRARY_IMPL(mxs_nf4, Meta, m) {
   m.impl("lora_bwd", &lora_bwd_meta);
   m.impl("lora_fwd_group", &lora_fwd_group_meta);
   m.impl("lora_bwd_group", &lora_bwd_group_meta);
+  m.impl("mlp_fwd", &mlp_fwd_meta);
+  m.impl("mlp_bwd", &mlp_bwd_meta);
 }
 
 // The autograd ops: the same node with or without grad mode (without it, or with no input

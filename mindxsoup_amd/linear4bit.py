@@ -621,6 +621,11 @@ def hip_forward(layer, x, original=None):
         if original is None:
             raise ValueError("input not supported by the HIP NF4 path")
         return original(layer, x)
+    return _direct(layer, x)
+
+
+def _direct(layer, x):
+    """The direct path's projection of an input _direct_ok accepts."""
     bias = _cast_bias_once(layer, x)
     if bias is not None:
         bias = bias.to(layer.compute_dtype)
@@ -717,7 +722,7 @@ class Linear4bit(torch.nn.Module):
         if isinstance(x, torch.Tensor) and x.is_cuda and stream.offloaded(self):
             return _streamed_forward(self, x)
         if _direct_ok(self, x):
-            return hip_forward(self, x)
+            return hip_forward(self, x) if cache_fp16 else _direct(self, x)
         return _generic_forward(self, x)
 
 

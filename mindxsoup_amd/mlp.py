@@ -23,7 +23,7 @@ SwiGLU reads it, as the separate kernel does, and both evaluate the same fp32 fo
 
 import torch
 
-from . import direct, kernels, linear4bit, peft_lora, stream
+from . import direct, kernels, linear4bit, ops, peft_lora, stream
 from .linear4bit import Proj as _Proj, _cast_bias_once, lora_backward_group
 from .silu_mul import silu_mul
 
@@ -46,6 +46,17 @@ class NF4LoraMLPFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x2d, ga, gb, ua, ub, da, db, projs):
         pg, pu, pd = projs
+        ctx.compiled = _compiled(projs)
+        if ctx.compiled:
+            train = not isinstance(ctx, direct._Unrecorded)
+            outs = ops.mlp_fwd(x2d, projs, [ga, ua, da], [gb, ub, db], train)
+            if train:
+                ctx.save_for_backward(x2d, *outs[1:])
+                # the byte masks are not kept: their bits are saved
+                ctx.projs = tuple(_Proj(p.packed, p.state, None, None, p.mask_scale, p.s)
+                                  for p in projs)
+                ctx.dtypes = tuple(t.dtype for t in (ga, gb, ua, ub, da, db))
+            return outs[0]
         M = x2d.shape[0]
         inter, hidden = pu.state.shape
         g_a, g_b, u_a, u_b, d_a, d_b = (t.to(torch.float16).contiguous()
@@ -88,6 +99,13 @@ class NF4LoraMLPFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
+        if ctx.compiled:
+            x2d, gate, up, h, *rest = ctx.saved_tensors
+            grads = ops.mlp_bwd(dy.to(torch.float16).contiguous(), x2d, gate, up, h, rest[9:],
+                                rest[:3], rest[3:6], rest[6:9], ctx.projs,
+                                ctx.needs_input_grad[:7])
+            return (grads[0], *(g if g is None or g.dtype == t else g.to(t)
+                                for g, t in zip(grads[1:], ctx.dtypes)), None)
         (x2d, gate, up, h, ht_g, at_g, bt_g, ht_u, at_u, bt_u, ht_d, at_d,
          bt_d) = ctx.saved_tensors
         pg, pu, pd = ctx.projs
@@ -128,6 +146,16 @@ class NF4LoraMLPFunction(torch.autograd.Function):
         return (dx, *grads, None)
 
 
+def _compiled(projs):
+    """Whether the block runs through torch.ops.mxs_nf4.mlp_fwd / mlp_bwd (the launch sequence
+    below in C++, the same bits; the Python sequence took 580 us of host time per training pass
+    on MI355X's host, longer than the GPU's 370 at 1024 tokens): the operator library is on and
+    gate and up share one scaling and dropout rate."""
+    pg, pu, _ = projs
+    return (ops.ENABLED and not GLU_FORWARD_TAIL and pg.s == pu.s
+            and pg.mask_scale == pu.mask_scale)
+
+
 def _is_fp16_4bit(linear):
     """A 4-bit projection computing in fp16: bitsandbytes' or this package's Linear4bit, bare or
     LoRA-wrapped (solution/mlp.py:21-24)."""
@@ -141,25 +169,33 @@ def fused_ok(mlp, x16):
     """Whether NF4LoraMLPFunction takes this MLP and fp16 input: every projection a LoRA layer
     with peft's layout (peft_lora.adapter_of) over an NF4 base that the fused kernels take,
     shaped hidden -> inter -> hidden."""
+    return _adapters(mlp, x16) is not None
+
+
+def _adapters(mlp, x16):
+    """The three projections' adapters where the fused block takes them (fused_ok), else None."""
     if not (FUSED_SWIGLU and linear4bit.FUSED_LORA and x16.dim() >= 2):
-        return False
+        return None
     ads = [peft_lora.adapter_of(getattr(mlp, n, None)) for n in _NAMES]
     if any(ad is None for ad in ads):
-        return False
+        return None
     states = [ad.base.weight.quant_state for ad in ads]
     inter, hidden = states[0].shape
     if tuple(states[1].shape) != (inter, hidden) or tuple(states[2].shape) != (hidden, inter):
-        return False
+        return None
     if any(stream.offloaded(ad.base) for ad in ads):
-        return False  # offloaded bases take each projection's streamed path
+        return None  # offloaded bases take each projection's streamed path
     h_probe = x16.new_empty((1, inter))  # down_proj's input: fp16 on the same device
-    return all(peft_lora.takes(ad, probe) for ad, probe in zip(ads, (x16, x16, h_probe)))
+    if all(peft_lora.takes(ad, probe) for ad, probe in zip(ads, (x16, x16, h_probe))):
+        return ads
+    return None
 
 
-def fused_forward(mlp, x16):
+def fused_forward(mlp, x16, ads=None):
     """NF4LoraMLPFunction on an MLP that fused_ok accepts (same dropout draws, in the same
-    order, as calling the three projections)."""
-    ads = [peft_lora.adapter_of(getattr(mlp, n)) for n in _NAMES]
+    order, as calling the three projections); ads: its adapters, when already resolved."""
+    if ads is None:
+        ads = [peft_lora.adapter_of(getattr(mlp, n)) for n in _NAMES]
     lead = x16.shape[:-1]
     x2d = x16.reshape(-1, x16.shape[-1]).contiguous()
     projs, tensors = [], []
@@ -168,8 +204,9 @@ def fused_forward(mlp, x16):
         keep, mask_scale = None, 1.0
         if ad.dropping():
             # gate and up read x; down reads hidden, [M, inter]
-            keep = kernels.keep_bits(ad.keep_mask(x2d, (x2d.shape[0], base.in_features)),
-                                     x2d.shape[0], base.in_features)
+            keep = ad.keep_mask(x2d, (x2d.shape[0], base.in_features))
+            if not ops.ENABLED:  # the operator packs them, gate's and up's in one launch
+                keep = kernels.keep_bits(keep, x2d.shape[0], base.in_features)
             mask_scale = 1.0 / (1.0 - ad.p)
         projs.append(_Proj(base.weight.data.view(-1, 1), base.weight.quant_state,
                            _cast_bias_once(base, x16), keep, mask_scale, ad.s))
@@ -191,8 +228,9 @@ def fp16_forward(mlp, x, previous=None):
             raise ValueError("input not supported by the fp16 MLP path")
         return previous(mlp, x)
     x16 = x.to(torch.float16)
-    if fused_ok(mlp, x16):
-        out = fused_forward(mlp, x16)
+    ads = _adapters(mlp, x16)
+    if ads is not None:
+        out = fused_forward(mlp, x16, ads)
     else:
         out = mlp.down_proj(silu_mul(mlp.gate_proj(x16), mlp.up_proj(x16)))
     return out.to(x.dtype)

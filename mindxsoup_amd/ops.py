@@ -20,7 +20,7 @@ from . import _lib
 PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libmxs_nf4_torch.so")
 
 OPS = ("dequant", "linear_fwd", "linear_bwd_dx", "lora_fwd", "lora_bwd", "lora_fwd_group",
-       "lora_bwd_group", "linear", "lora_linear", "lora_siblings")
+       "lora_bwd_group", "linear", "lora_linear", "lora_siblings", "mlp_fwd", "mlp_bwd")
 
 # set by apply() from FEATURES["torch_ops"]; False: the Python Functions.  Off when MXS_NF4_LIB
 # names another build of the C-ABI library: this library links the package's own copy by file
@@ -80,6 +80,28 @@ def lora_siblings(x2d, projs, lora_as, lora_bs, one_gemm=True, rope=None):
         [p.state.state2.absmax for p in projs], [p.state.offset for p in projs],
         [p.bias for p in projs], [p.keep for p in projs], float(p0.mask_scale), float(p0.s),
         bool(one_gemm), cos, sin, int(n_rope))
+
+
+def _nf4_lists(projs):
+    """The five NF4 operand lists of several projections (linear4bit.Proj)."""
+    return list(map(list, zip(*(nf4(p.packed, p.state) for p in projs))))
+
+
+def mlp_fwd(x2d, projs, lora_as, lora_bs, train):
+    """The MLP block's forward launches (mlp.NF4LoraMLPFunction) for gate, up and down, gate and
+    up with one scaling and dropout rate: [y], or with train [y, gate, up, h, three ht, three at,
+    three bt, three keep bits (None without dropout)]."""
+    return load().mlp_fwd(x2d, lora_as, lora_bs, *_nf4_lists(projs), [p.bias for p in projs],
+                          [p.keep for p in projs], [float(p.mask_scale) for p in projs],
+                          [float(p.s) for p in projs], train)
+
+
+def mlp_bwd(dy, x2d, gate, up, h, keeps, hts, ats, bts, projs, wants):
+    """Its backward launches: [dx, dA and dB of gate, up and down] (None where not wanted); gate
+    and up are overwritten with their gradients."""
+    return load().mlp_bwd(dy, x2d, gate, up, h, keeps, hts, ats, bts, *_nf4_lists(projs),
+                          [float(p.mask_scale) for p in projs], [float(p.s) for p in projs],
+                          [int(bool(w)) for w in wants])
 
 
 def dequant(packed, shape, dtype, absmax_8bit=None, code=None, absmax2=None, offset=None,

@@ -1,0 +1,54 @@
+"""The MLP block through torch.ops.mxs_nf4.mlp_fwd / mlp_bwd against the Python launch sequence: the
+same kernels in the same order, so output and gradients are equal bit for bit."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _mlp(dev, hidden, inter, r, dropout):
+    from mindxsoup_amd.linear4bit import Linear4bit, LoraLinear4bit
+    from mindxsoup_amd.mlp import MLP
+
+    layers = []
+    for n, k in ((inter, hidden), (inter, hidden), (hidden, inter)):
+        base = Linear4bit.from_weight((torch.randn((n, k), device=dev) * 0.02).half())
+        layers.append(LoraLinear4bit(base, r=r, lora_alpha=2 * r, lora_dropout=dropout))
+        torch.nn.init.normal_(layers[-1].lora_B["default"].weight, std=0.02)
+    return MLP(*layers)
+
+
+@pytest.mark.parametrize("M,hidden,inter,r,dropout,frozen", [
+    (5, 1536, 8960, 16, 0.0, ()), (37, 1536, 8960, 16, 0.05, ()),
+    (300, 1536, 4224, 32, 0.05, ("gate_proj", "x")), (1024, 1536, 8960, 16, 0.05, ("down_proj",)),
+    (130, 1536, 1536, 16, 0.05, ())])
+def test_compiled_block_equals_python_sequence(cuda, monkeypatch, M, hidden, inter, r, dropout,
+                                               frozen):
+    from mindxsoup_amd import ops
+
+    print(f"case mlp op M={M} inter={inter} r={r} frozen={frozen}", flush=True)
+    torch.manual_seed(M)
+    mlp = _mlp(cuda, hidden, inter, r, dropout).train()
+    for name in frozen:
+        if name != "x":
+            for p in getattr(mlp, name).parameters():
+                p.requires_grad_(False)
+    x = torch.randn((1, M, hidden), device=cuda)
+    dy = torch.randn((1, M, hidden), device=cuda) * 1e-2
+    got = {}
+    for enabled in (True, False):
+        monkeypatch.setattr(ops, "ENABLED", enabled)
+        mlp.zero_grad(set_to_none=True)
+        torch.manual_seed(7)  # the same dropout draws
+        xl = x.clone().requires_grad_("x" not in frozen)
+        y = mlp(xl)
+        y.backward(dy)
+        with torch.no_grad():
+            mlp.eval()
+            e = mlp(x)
+            mlp.train()
+        got[enabled] = [y.detach(), e, xl.grad] + [p.grad for p in mlp.parameters()]
+    for i, (a, b) in enumerate(zip(got[True], got[False])):
+        assert (a is None) == (b is None), i
+        assert a is None or torch.equal(a, b), i
