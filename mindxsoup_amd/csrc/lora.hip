@@ -407,12 +407,25 @@ static int waves_for(int steps) {
 }
 
 // Reduction slices for the rows kernel: one (a single launch) unless the reduction is long
-// (>= 1024) and a workspace is given; then enough slices for about 256 workgroups, at most 4.
+// (>= 1024) and a workspace is given; then enough slices for about 256 workgroups, at most 4, and
+// more where they fill the last round of the 256 CUs: rounds / slices is the launch's length in
+// unsliced workgroups.  3001 tokens are 188 row blocks, one round in one slice and 3/4 of that in
+// four (gate/up's dHs 36.0 -> 25.6 us, their Hs 12.8 -> 11.2, down's Hs 28.4 -> 27.5), 6144 tokens
+// 384, two rounds or 3/2 in two slices (52.0 -> 43.1, 19.9 -> 15.6, 53.9 -> 46.1).
 static int rows_slices(int K, int ldt) {
   if (K < 1024) return 1;
   const int row_blocks = (ldt + 15) / 16;
-  int sl = 256 / row_blocks;
-  return sl < 1 ? 1 : sl > 4 ? 4 : sl;
+  const int sl = 256 / row_blocks;
+  int best = sl < 1 ? 1 : sl > 4 ? 4 : sl;
+  double length = (double)((row_blocks * best + 255) / 256) / best;
+  for (int s : {2, 4}) {
+    const double l = (double)((row_blocks * s + 255) / 256) / s;
+    if (s > best && l < 0.9 * length) {
+      best = s;
+      length = l;
+    }
+  }
+  return best;
 }
 
 // Slices and waves of one rows problem.  The workspace size query assumes ldt = M rounded up
