@@ -2436,7 +2436,7 @@ struct DensePlan {
 // What the dense route and the fused kernels cost, in microseconds on MI355X (HIP graphs, M = 1024
 // to 8192, the projections' shapes): rounds of tiles over the CUs times a tile's time, which is a
 // K-step's time (power-limited when every CU multiplies) plus what stands alone at its ends.  The
-// route is taken where its estimate is 5 % below the fused kernels'.  Measured / estimated, dense
+// route is taken where its estimate is 3 % below the fused kernels'.  Measured / estimated, dense
 // against fused: down_proj forward at 8192 tokens 220 / 228 against 370, at 3001 105 / 104 against
 // 128, at 2048 80 / 79 against 88; its dX (8960 wide) 244 / 247 against 267 at 8192, 68 / 66
 // against 75 at 2048, not taken at 3001 (113 / 129 against 112); 1536 x 1536 at 8192 49 / 47
@@ -2444,7 +2444,7 @@ struct DensePlan {
 static double fused_tile_us(int cfg, int steps) {
   switch (cfg) {
     case 6: return 0.95 * steps + 7.0;             // 256x128
-    case 7: return 1.15 * steps + 8.0;             // 256x160
+    case 7: return 1.20 * steps + 8.4;             // 256x160
     case 9: case 11: return 0.87 * steps + 8.0;    // 256x96
     case 10: return 0.60 * steps + 6.5;            // 128x128
     default: return 0.41 * steps + 4.7;            // 128x64
@@ -2454,6 +2454,23 @@ static double fused_tile_us(int cfg, int steps) {
 static double dense_tile_us(int bn, int steps) {
   const double step = bn == 320 ? 1.78 : bn == 256 ? 1.47 : 1.32;
   return step * steps + 13.0;
+}
+
+// `wgs` workgroups of t microseconds on the CUs; the last, partial round runs with idle CUs: an
+// unloaded chip takes `alone` of t.
+static double rounds_us(int64_t wgs, int cus, double t, double alone) {
+  const int64_t full = wgs / cus;
+  const double part = (double)(wgs % cus) / cus;
+  return full * t + (part > 0 ? t * (alone + (1.0 - alone) * part) : 0.0);
+}
+constexpr double kFusedAlone = 0.75, kDenseAlone = 0.87;
+
+// The SwiGLU adjoint's gate / up traffic behind a GEMM's tiles: its working set of two [M, Nc]
+// buffers in the 256 MB cache (21 us at 3001 tokens) or past it (8192 tokens: fused 79, dense
+// 108).
+static double glu_us(int M, int Nc, bool dense) {
+  const double values = (double)M * Nc;
+  return values * (values < 32e6 ? 0.8e-6 : dense ? 1.47e-6 : 1.08e-6);
 }
 
 static double reduce_us(int splits, int M, int Nc) {
@@ -2467,10 +2484,9 @@ static double fused_us(int M, int Nc, int Kr, bool bwd, bool glu) {
   choose(M, Nc, Kr, bwd, &cfg, &sp);
   if (cfg < 6) return -1.0;
   const int64_t tiles = ceil_div(M, kWsBM[cfg - 6]) * ceil_div(Nc, kWsBN[cfg - 6]) * sp;
-  const double tail = glu ? 11.3 : 0.0;  // the SwiGLU's gate / up traffic, per round
-  return ceil_div(tiles, cu_count()) *
-             (fused_tile_us(cfg, (int)ceil_div(Kr / kBK, sp)) + tail) +
-         reduce_us(sp, M, Nc);
+  return rounds_us(tiles, cu_count(), fused_tile_us(cfg, (int)ceil_div(Kr / kBK, sp)),
+                   kFusedAlone) +
+         reduce_us(sp, M, Nc) + (glu ? glu_us(M, Nc, false) : 0.0);
 }
 
 // The best dense plan for n problems [M, Nc[i]] over `steps` K-steps (sum: one output Nc[0] and
@@ -2490,9 +2506,9 @@ static double dense_us(int M, int n, const int* Nc, int steps, int64_t values, b
       if (sp > 1 && (w == 320 || (n > 1 && !sum) || steps / sp < 12)) break;
       const int per = (int)ceil_div(steps, sp);
       if (ceil_div(steps, per) != sp) continue;
-      const double t = ceil_div(tiles * sp, cus) *
-                           (dense_tile_us(w, per) + (glu ? 0.09 * w : 0.0)) +
-                       reduce_us(sp, M, Nc[0]) + 2.53 * values / 4.2e6 + 1.5;
+      const double t = rounds_us(tiles * sp, cus, dense_tile_us(w, per), kDenseAlone) +
+                       (glu ? glu_us(M, Nc[0], true) : 0.0) + reduce_us(sp, M, Nc[0]) +
+                       2.53 * values / 4.2e6 + 1.5;
       if (best < 0 || t < best) {
         best = t;
         d->bn = w;
@@ -2527,7 +2543,7 @@ static bool dense_plan(int M, int Nc, int Kr, bool bwd, bool glu, DensePlan* d) 
     const double f = fused_us(M, Nc, Kr, bwd, glu);
     if (f < 0) return false;
     const double t = dense_us(M, 1, &Nc, Kr / kBK, (int64_t)Nc * Kr, false, glu, 0, p);
-    return t > 0 && t < 0.95 * f;
+    return t > 0 && t < 0.97 * f;
   });
 }
 
@@ -3143,11 +3159,11 @@ static bool dense_pair_plan(int M, const int N[2], int K, DensePlan* d) {
       longest = std::max(longest, N[i] / kBK);
     }
     const int sp = pair_splits(M, N, K);
-    const double f = ceil_div(ceil_div(M, 256) * ceil_div(K, 96) * 2 * sp, cus) *
-                         fused_tile_us(11, (int)ceil_div(longest, sp)) +
+    const double f = rounds_us(ceil_div(M, 256) * ceil_div(K, 96) * 2 * sp, cus,
+                               fused_tile_us(11, (int)ceil_div(longest, sp)), kFusedAlone) +
                      reduce_us(2 * sp, M, K);
     const double t = dense_us(M, 2, &K, steps, weight_values(2, N, K), true, false, 0, p);
-    return t > 0 && t < 0.95 * f;
+    return t > 0 && t < 0.97 * f;
   });
 }
 
@@ -3161,10 +3177,10 @@ static bool dense_sum_plan(int n, int M, const int* N, int K, DensePlan* d) {
   return dense_memo(key, d, [&](DensePlan* p) {
     int steps = 0;
     for (int i = 0; i < n; i++) steps += N[i] / kBK;
-    const double f = ceil_div(ceil_div(M, 128) * ceil_div(K, 128), cus) *
-                     (fused_tile_us(10, steps) + 8.0);
+    const double f = rounds_us(ceil_div(M, 128) * ceil_div(K, 128), cus,
+                               fused_tile_us(10, steps) + 8.0, kFusedAlone);
     const double t = dense_us(M, n, &K, steps, weight_values(n, N, K), true, false, 0, p);
-    return t > 0 && t < 0.95 * f;
+    return t > 0 && t < 0.97 * f;
   });
 }
 
@@ -3189,11 +3205,11 @@ static bool dense_group_plan(int n, int M, const int* N, int K, bool rope, Dense
     }
     const int steps = K / kBK;
     const double f = wide && !rope
-        ? 0.95 * ceil_div(tiles160, cus) * fused_tile_us(7, steps)
-        : ceil_div(tiles128, cus) * (fused_tile_us(10, steps) + (rope ? 5.5 : 0.0));
+        ? 0.95 * rounds_us(tiles160, cus, fused_tile_us(7, steps), kFusedAlone)
+        : rounds_us(tiles128, cus, fused_tile_us(10, steps) + (rope ? 5.5 : 0.0), kFusedAlone);
     const double t = dense_us(M, n, N, steps, weight_values(n, N, K), false, false, rope ? 256 : 0,
                               p);
-    return t > 0 && t < 0.95 * f;
+    return t > 0 && t < 0.97 * f;
   });
 }
 
