@@ -59,6 +59,10 @@ class NF4LoraMLPFunction(torch.autograd.Function):
             return outs[0]
         M = x2d.shape[0]
         inter, hidden = pu.state.shape
+        # packed once: every launch below and the backward's read the bits
+        projs = pg, pu, pd = tuple(
+            _Proj(p.packed, p.state, p.bias, kernels.keep_bits(p.keep, M, p.state.shape[1]),
+                  p.mask_scale, p.s) for p in projs)
         g_a, g_b, u_a, u_b, d_a, d_b = (t.to(torch.float16).contiguous()
                                         for t in (ga, gb, ua, ub, da, db))
         # gate's and up's LoRA row products read the same x: one launch when they can share it
@@ -205,8 +209,6 @@ def fused_forward(mlp, x16, ads=None):
         if ad.dropping():
             # gate and up read x; down reads hidden, [M, inter]
             keep = ad.keep_mask(x2d, (x2d.shape[0], base.in_features))
-            if not ops.ENABLED:  # the operator packs them, gate's and up's in one launch
-                keep = kernels.keep_bits(keep, x2d.shape[0], base.in_features)
             mask_scale = 1.0 / (1.0 - ad.p)
         projs.append(_Proj(base.weight.data.view(-1, 1), base.weight.quant_state,
                            _cast_bias_once(base, x16), keep, mask_scale, ad.s))

@@ -52,3 +52,21 @@ def test_compiled_block_equals_python_sequence(cuda, monkeypatch, M, hidden, int
     for i, (a, b) in enumerate(zip(got[True], got[False])):
         assert (a is None) == (b is None), i
         assert a is None or torch.equal(a, b), i
+
+
+def test_unequal_scalings_pack_masks_once(cuda, monkeypatch):
+    """gate and up with scalings of their own take the Python sequence: each byte keep mask is
+    packed once for the forward's launches and the backward's."""
+    from mindxsoup_amd import kernels
+
+    print("case mlp unequal scalings", flush=True)
+    packed, pack = [], kernels.keep_bits
+    monkeypatch.setattr(kernels, "keep_bits", lambda m, M, K: (
+        packed.append((M, K)) if m is not None and m.dtype != torch.int32 else None) or pack(m, M, K))
+    torch.manual_seed(3)
+    mlp = _mlp(cuda, 1536, 2048, 16, 0.05).train()
+    mlp.up_proj.scaling["default"] = 1.0
+    x = torch.randn((1, 37, 1536), device=cuda, requires_grad=True)
+    y = mlp(x)
+    y.backward(torch.randn_like(y))
+    assert packed == [(37, 1536), (37, 1536), (37, 2048)]
