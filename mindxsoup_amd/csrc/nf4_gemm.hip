@@ -2678,6 +2678,8 @@ static int gemm_entry(bool bwd, const GemmArgs& a, int cfg, int splits, hipStrea
         dense_takes(a.M, a.Nc, a.Kr) && dense_plan(a.M, a.Nc, a.Kr, bwd, a.glu == 2, &d))
       return launch_dense(bwd, &a, 1, false, d, a.ws, true, nullptr, stream);
     choose(a.M, a.Nc, a.Kr, bwd, &cfg, &splits);
+    // no workspace for a split of few tokens: the shape's own plan, where that has none
+    if (splits > 1 && !a.ws) choose_base(a.M, a.Nc, a.Kr, bwd, &cfg, &splits);
   }
   if (cfg >= kNumCfg || cfg == 5) return MXS_ERR_ARG;
   return bwd ? launch_by_id<true>(cfg, a, splits, stream)

@@ -75,3 +75,19 @@ def test_pair_and_glu_equal_single_launches(cuda, M):
     y = torch.empty_like(up)
     kernels.nf4_linear_fwd_noalloc(x, ws[0][0], ws[0][1], y)
     assert torch.equal(y, kernels.nf4_linear_fwd(x, ws[0][0], ws[0][1]))
+
+
+def test_split_plan_without_a_workspace(cuda):
+    """A wide, long projection splits at few tokens; a caller without a workspace gets the plan
+    that needs none."""
+    from mindxsoup_amd import _lib, kernels
+    from mindxsoup_amd.quant import quantize_4bit
+
+    M, k, n = 64, 11008, 4096
+    print("case split plan without a workspace", flush=True)
+    packed, st = quantize_4bit((torch.randn((n, k), device=cuda) * 0.02).half())
+    x = torch.randn((M, k), device=cuda).half()
+    y = torch.empty((M, n), device=cuda, dtype=torch.float16)
+    _lib.call("mxs_nf4_linear_fwd", _lib.ptr(x), M, k, n, *kernels._nf4_args(packed, st), None,
+              None, None, 0, _lib.ptr(y), None, -1, 1, _lib.stream_of(x.device))
+    _close(y, kernels.nf4_linear_fwd(x, packed, st))
