@@ -334,7 +334,6 @@ __device__ __forceinline__ void dense_tile(const GemmArgs* as, int nsum, int bx,
   // accumulator start: bias and the LoRA term (first split), its operands staged in stage 1
   const bool lora = (int)blockIdx.z == a.zf && (a.lora_hp || a.lora_h);
   const bool lora16 = lora && a.r == 16;
-  const bool kmask = BWD && lora && a.mask;
   using MS = MaskStage<BM, BN, NT>;
   constexpr int LSH = (BM + BN) * 16;
   static_assert(LSH * 2 + BM * MS::KST <= (int)STAGE, "staged operands fit a stage");
@@ -343,6 +342,9 @@ __device__ __forceinline__ void dense_tile(const GemmArgs* as, int nsum, int bx,
   float16_t acc[TM][TN];
   AccStart<TM, TN, BWD> start;
   auto begin = [&](const GemmArgs& p, float16_t (&c)[TM][TN]) {
+    // of summed problems any may have keep bits and any none; uniform over the workgroup, so its
+    // waves meet at the same barriers
+    const bool kmask = BWD && lora && p.mask;
     if (lora16 || kmask) {
       LoraStage<BM, BN, NT> lst;
       MS mst;

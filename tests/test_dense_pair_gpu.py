@@ -1,0 +1,68 @@
+"""The summed input gradient of gate and up from decoded weights (k_dense_gemm over two reductions,
+mxs_nf4_linear_bwd_dx_hp_pair at many tokens): each projection's own keep mask or none, ranks
+staged through LDS (16) and read from memory, unequal widths.
+
+Reference: the two projections' single input gradients on the fused kernels, each rounded to fp16,
+added in fp32.  The summed launch rounds once, so the two differ by the parts' roundings (half an
+ulp each), its own, and the fp32 sums' other order (2^-18 of the largest value)."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+S, MS = 2.0, 1 / 0.95
+K = 1536
+
+
+def _proj(dev, n, M, r, seed):
+    from mindxsoup_amd.quant import quantize_4bit
+
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    rnd = lambda *s: torch.randn(s, device=dev, generator=g)  # noqa: E731
+    packed, st = quantize_4bit((rnd(n, K) * 0.02).half())
+    return dict(n=n, packed=packed, st=st, a=(rnd(r, K) / K ** 0.5).half(),
+                b=(rnd(n, r) * 0.01).half(), dy=rnd(M, n).half(), ht=rnd(r, (M + 7) // 8 * 8).half(),
+                keep=(torch.rand((M, K), device=dev, generator=g) >= 0.05).to(torch.uint8))
+
+
+def _bound(parts, two):
+    return 2.0 ** -11 * (sum(t.float().abs() for t in parts) + two.abs()) * 1.01 + \
+        2.0 ** -18 * two.abs().max()
+
+
+@pytest.mark.parametrize("widths", [(8960, 8960), (8960, 6144)])
+@pytest.mark.parametrize("r", [16, 32, 64])
+@pytest.mark.parametrize("masked", [(True, False), (False, True), (False, False), (True, True)])
+def test_masks_of_either_projection(cuda, masked, r, widths):
+    from mindxsoup_amd import _lib, kernels
+
+    M = 1430  # the last row band holds 150 rows
+    print(f"case dense dX pair masked={masked} r={r} widths={widths}", flush=True)
+    nbytes = _lib.lib().mxs_nf4_linear_bwd_dx_pair_workspace_bytes(M, *widths, K)
+    if nbytes < 2 * sum(widths) * K:  # room for the decoded weights: the dense route
+        pytest.skip("this device's CU count plans the fused kernel")
+    ps = [_proj(cuda, n, M, r, 20 + i) for i, n in enumerate(widths)]
+    keeps = [p["keep"] if m else None for p, m in zip(ps, masked)]
+    dhps = [kernels.lora_dh_partials(p["dy"], p["b"].t().contiguous(), S) for p in ps]
+    ats = [p["a"].t().contiguous() for p in ps]
+    dys = [p["dy"] for p in ps]
+    nf4 = ([p["packed"] for p in ps], [p["st"] for p in ps])
+    dx, dhts = kernels.nf4_linear_bwd_dx_hp_pair(dys, *nf4, dhps, ats, keeps, MS)
+    parts = [kernels.nf4_linear_bwd_dx_hp(d, p["packed"], p["st"], h, at, kp, MS, cfg=11,
+                                          splits=4)
+             for d, p, h, at, kp in zip(dys, ps, dhps, ats, keeps)]
+    two = parts[0][0].float() + parts[1][0].float()
+    assert bool(((dx.float() - two).abs() <= _bound([t[0] for t in parts], two)).all())
+    for (_, want), dht in zip(parts, dhts):
+        assert torch.equal(dht, want)
+    if widths[0] != widths[1]:  # one launch for both gradients needs equal widths
+        return
+    x, hts = torch.randn((M, K), device=cuda).half(), [p["ht"] for p in ps]
+    dx2, dhts2, grads = kernels.nf4_linear_bwd_dx_hp_pair_grads(dys, *nf4, dhps, ats, hts, x,
+                                                                keeps, MS)
+    assert torch.equal(dx, dx2)
+    for (da, db), p, dht, ht, kp in zip(grads, ps, dhts2, hts, keeps):
+        da1, db1 = kernels.lora_grads(dht, ht, x, p["dy"], kp, MS)
+        assert torch.equal(da, da1) and torch.equal(db, db1)
