@@ -198,12 +198,16 @@ int mxs_nf4_linear_bwd_dx_hp(const void* dy, int M, int N, int K, const void* pa
  * with dX_i = dY_i . W_i + mask_i * mask_scale * (fp16(sum of lora_dhp_i) . lora_at_i^T), as
  * mxs_nf4_linear_bwd_dx_hp computes each.  These are the gate and up projections of the MLP
  * (solution/mlp.py:42-43), whose input gradients autograd adds for their shared input.  ONE
- * launch of the split-K kernel runs both reductions (each split two ways) and one reduce adds
- * the four fp32 partial planes in order, so neither dX_i is rounded to fp16 on its own; the
- * result equals the fp32 sum of the two GEMMs rounded once.  Arrays hold the per-projection
- * arguments (N[i] = out_features; mask and lora_dht may be NULL, or any entry); the two share
- * M, K, r, ldt, hp_slices and mask_scale.  workspace: at least
- * mxs_nf4_linear_bwd_dx_pair_workspace_bytes(M, N[0], N[1], K) bytes.  Only where
+ * launch of the split-K kernel runs both reductions (each split two ways, up to eight where one
+ * or two row bands would leave CUs idle) and one reduce adds the fp32 partial planes in order; at
+ * many tokens, where that costs less, both weights are decoded to fp16 in the workspace and one
+ * plain GEMM runs the two reductions into one accumulator (split over a few planes where the
+ * tiles are few).  Either way neither dX_i is rounded to fp16 on its own; the result equals the
+ * fp32 sum of the two GEMMs rounded once.  Arrays hold the per-projection arguments (N[i] =
+ * out_features; mask and lora_dht may be NULL, or any entry); the two share M, K, r, ldt,
+ * hp_slices and mask_scale.  workspace: at least
+ * mxs_nf4_linear_bwd_dx_pair_workspace_bytes(M, N[0], N[1], K) bytes (the decoded weights are
+ * used only where it is 16-byte aligned).  Only where
  * mxs_nf4_linear_bwd_dx_pair_ok(M, N[0], N[1], K) is 1 (both projections plan the narrow-output
  * split-K kernel on their own), else MXS_ERR_SIZE. */
 int mxs_nf4_linear_bwd_dx_hp_pair(const void* const dy[2], int M, const int N[2], int K,
@@ -222,9 +226,9 @@ int mxs_nf4_linear_bwd_dx_hp_pair(const void* const dy[2], int M, const int N[2]
  * LoRA branches (peft's lora_A / lora_B under solution/mlp.py:42-43) with their summed input
  * gradient.  Two launches instead of three: the pair GEMM, then one launch for its split-K
  * reduce and the gradients (independent of each other), the reduce's workgroups filling the
- * CUs the gradients' last partial round leaves idle.  Same conditions as
- * mxs_nf4_linear_bwd_dx_hp_pair, and the two projections share their gradients' columns per
- * lane (as mxs_lora_grads_group requires). */
+ * CUs the gradients' last partial round leaves idle (the gradients alone where dX came from one
+ * unsplit plane).  Same conditions as mxs_nf4_linear_bwd_dx_hp_pair, and the two projections
+ * share their gradients' columns per lane (as mxs_lora_grads_group requires). */
 int mxs_nf4_linear_bwd_dx_hp_pair_grads(
     const void* const dy[2], int M, const int N[2], int K, const void* const packed[2],
     const void* const absmax8[2], const float* const code[2], const float* const absmax2[2],
@@ -232,6 +236,18 @@ int mxs_nf4_linear_bwd_dx_hp_pair_grads(
     const void* const lora_at[2], int r, const void* const mask[2], float mask_scale,
     void* const lora_dht[2], const void* const ht[2], const void* x, float* const da[2],
     float* const db[2], void* dx, void* workspace, hipStream_t stream);
+
+/* mxs_nf4_linear_bwd_dx_hp_pair (ht, x, da and db NULL) or mxs_nf4_linear_bwd_dx_hp_pair_grads
+ * within a workspace of workspace_bytes: the plan those entries run where it fits, else the fused
+ * launch with each reduction split two ways, which takes 16 * M * K bytes; fewer are refused
+ * (MXS_ERR_SIZE).  The plans differ in the order of the fp32 sums. */
+int mxs_nf4_linear_bwd_dx_hp_pair_ws(
+    const void* const dy[2], int M, const int N[2], int K, const void* const packed[2],
+    const void* const absmax8[2], const float* const code[2], const float* const absmax2[2],
+    const float* const offset[2], const float* const lora_dhp[2], int hp_slices, int ldt,
+    const void* const lora_at[2], int r, const void* const mask[2], float mask_scale,
+    void* const lora_dht[2], const void* const ht[2], const void* x, float* const da[2],
+    float* const db[2], void* dx, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
 /* Two projections over the same input x [M, K] (the gate and up projections of the MLP,
  * solution/mlp.py:42-43, each NF4LinearFunction.forward of solution/linear4bit.py:47-49 with

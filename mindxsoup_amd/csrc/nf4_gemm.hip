@@ -3169,6 +3169,27 @@ static bool dense_pair_plan(int M, const int N[2], int K, DensePlan* d) {
   });
 }
 
+// The pair's plan within a caller's workspace: decoded weights where planned and the bytes (and
+// their alignment) are there, else the fused launch with its planned splits, else with two (four
+// planes, the least any caller brings).
+struct PairPlan {
+  bool dense;
+  DensePlan d;
+  int splits;
+};
+
+static int64_t pair_planes_bytes(int M, int K, int splits) {
+  return (int64_t)2 * splits * M * K * (int64_t)sizeof(float);
+}
+
+static bool pair_plan(int M, const int N[2], int K, const void* ws, int64_t bytes, PairPlan* p) {
+  p->dense = dense_pair_plan(M, N, K, &p->d) && (uintptr_t)ws % 16 == 0 &&
+             dense_sum_bytes(2, M, N, K, p->d) <= bytes;
+  p->splits = pair_splits(M, N, K);
+  if (pair_planes_bytes(M, K, p->splits) > bytes) p->splits = 2;
+  return p->dense || pair_planes_bytes(M, K, p->splits) <= bytes;
+}
+
 // q, k and v's summed dX without their gradients (against one launch of 128x128 tiles): 84 us
 // and 5 us of decode against 110 at 8192 tokens.
 static bool dense_sum_plan(int n, int M, const int* N, int K, DensePlan* d) {
@@ -3792,44 +3813,26 @@ int mxs_nf4_linear_bwd_dx_pair_ok(int M, int N0, int N1, int K) {
 int64_t mxs_nf4_linear_bwd_dx_pair_workspace_bytes(int M, int N0, int N1, int K) {
   if (!pair_plan_ok(M, N0, N1, K)) return 0;
   const int N[2] = {N0, N1};
-  const int64_t fused = (int64_t)2 * pair_splits(M, N, K) * M * K * (int64_t)sizeof(float);
+  const int64_t fused = pair_planes_bytes(M, K, pair_splits(M, N, K));
   DensePlan d;
   return dense_pair_plan(M, N, K, &d) ? std::max(fused, dense_sum_bytes(2, M, N, K, d)) : fused;
 }
 
-int mxs_nf4_linear_bwd_dx_hp_pair(const void* const dy[2], int M, const int N[2], int K,
-                                  const void* const packed[2], const void* const absmax8[2],
-                                  const float* const code[2], const float* const absmax2[2],
-                                  const float* const offset[2], const float* const lora_dhp[2],
-                                  int hp_slices, int ldt, const void* const lora_at[2], int r,
-                                  const void* const mask[2], float mask_scale,
-                                  void* const lora_dht[2], void* dx, void* workspace,
-                                  hipStream_t stream) {
-  GemmArgs p[2];
-  const int c = dx_pair_args(dy, M, N, K, packed, absmax8, code, absmax2, offset, lora_dhp,
-                             hp_slices, ldt, lora_at, r, mask, mask_scale, lora_dht, dx,
-                             workspace, p);
-  if (c != MXS_OK) return c == 1 ? MXS_OK : c;
-  DensePlan d;
-  if (dense_pair_plan(M, N, K, &d) && (uintptr_t)workspace % 16 == 0)
-    return launch_dense(true, p, 2, true, d, workspace, true, nullptr, stream);
-  return launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], pair_splits(M, N, K), stream);
-}
-
-int mxs_nf4_linear_bwd_dx_hp_pair_grads(
+int mxs_nf4_linear_bwd_dx_hp_pair_ws(
     const void* const dy[2], int M, const int N[2], int K, const void* const packed[2],
     const void* const absmax8[2], const float* const code[2], const float* const absmax2[2],
     const float* const offset[2], const float* const lora_dhp[2], int hp_slices, int ldt,
     const void* const lora_at[2], int r, const void* const mask[2], float mask_scale,
     void* const lora_dht[2], const void* const ht[2], const void* x, float* const da[2],
-    float* const db[2], void* dx, void* workspace, hipStream_t stream) {
-  if (!lora_dht || !ht || !x || !da || !db) return MXS_ERR_ARG;
+    float* const db[2], void* dx, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+  const bool grads = ht != nullptr;
+  if (grads && (!lora_dht || !x || !da || !db)) return MXS_ERR_ARG;
   GemmArgs p[2];
   const int c = dx_pair_args(dy, M, N, K, packed, absmax8, code, absmax2, offset, lora_dhp,
                              hp_slices, ldt, lora_at, r, mask, mask_scale, lora_dht, dx,
                              workspace, p);
   if (c == 1) {  // no tokens: dX is empty, dA and dB are empty reductions (zeros)
-    for (int i = 0; i < 2; i++) {
+    for (int i = 0; grads && i < 2; i++) {
       const int e = mxs_lora_grads(nullptr, nullptr, ldt, nullptr, nullptr, 0, K, N[i], r,
                                    nullptr, mask_scale, da[i], db[i], nullptr, stream);
       if (e != MXS_OK) return e;
@@ -3837,6 +3840,12 @@ int mxs_nf4_linear_bwd_dx_hp_pair_grads(
     return MXS_OK;
   }
   if (c != MXS_OK) return c;
+  PairPlan plan;
+  if (!pair_plan(M, N, K, workspace, workspace_bytes, &plan)) return MXS_ERR_SIZE;
+  if (!grads)
+    return plan.dense
+        ? launch_dense(true, p, 2, true, plan.d, workspace, true, nullptr, stream)
+        : launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], plan.splits, stream);
   if (r % 16) return MXS_ERR_SIZE;
   ColsGroup g{};
   g.n = 2;
@@ -3847,25 +3856,51 @@ int mxs_nf4_linear_bwd_dx_hp_pair_grads(
     if (e != MXS_OK) return e;
     if (cols_cpl(K + N[i]) != cpl) return MXS_ERR_SIZE;
   }
-  const int sp = pair_splits(M, N, K);
-  int planes = 2 * sp;
-  DensePlan d;
-  if (dense_pair_plan(M, N, K, &d) && (uintptr_t)workspace % 16 == 0) {
-    const int e = launch_dense(true, p, 2, true, d, workspace, false, &p[0].ws, stream);
+  int planes = 2 * plan.splits;
+  if (plan.dense) {
+    const int e = launch_dense(true, p, 2, true, plan.d, workspace, false, &p[0].ws, stream);
     if (e != MXS_OK) return e;
-    planes = d.splits;
+    planes = plan.d.splits;
     if (planes == 1)  // dX is complete: the gradients alone
       return mxs_lora_grads_group(2, lora_dht, ht, ldt, std::array<const void*, 2>{x, x}.data(),
                                   dy, M, std::array<int, 2>{K, K}.data(), N, r, mask, mask_scale,
                                   da, db, stream);
   } else {
     const int e =
-        launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], sp, stream, false);
+        launch_ws_pair<256, 96, 4, 1, true, 8, 5>(p[0], p[1], plan.splits, stream, false);
     if (e != MXS_OK) return e;
   }
   if (cpl == 8) return reduce_cols_launch<8>(p[0], planes, g, M, ldt, r, stream);
   if (cpl == 4) return reduce_cols_launch<4>(p[0], planes, g, M, ldt, r, stream);
   return reduce_cols_launch<2>(p[0], planes, g, M, ldt, r, stream);
+}
+
+int mxs_nf4_linear_bwd_dx_hp_pair(const void* const dy[2], int M, const int N[2], int K,
+                                  const void* const packed[2], const void* const absmax8[2],
+                                  const float* const code[2], const float* const absmax2[2],
+                                  const float* const offset[2], const float* const lora_dhp[2],
+                                  int hp_slices, int ldt, const void* const lora_at[2], int r,
+                                  const void* const mask[2], float mask_scale,
+                                  void* const lora_dht[2], void* dx, void* workspace,
+                                  hipStream_t stream) {
+  return mxs_nf4_linear_bwd_dx_hp_pair_ws(dy, M, N, K, packed, absmax8, code, absmax2, offset,
+                                          lora_dhp, hp_slices, ldt, lora_at, r, mask, mask_scale,
+                                          lora_dht, nullptr, nullptr, nullptr, nullptr, dx,
+                                          workspace, INT64_MAX, stream);
+}
+
+int mxs_nf4_linear_bwd_dx_hp_pair_grads(
+    const void* const dy[2], int M, const int N[2], int K, const void* const packed[2],
+    const void* const absmax8[2], const float* const code[2], const float* const absmax2[2],
+    const float* const offset[2], const float* const lora_dhp[2], int hp_slices, int ldt,
+    const void* const lora_at[2], int r, const void* const mask[2], float mask_scale,
+    void* const lora_dht[2], const void* const ht[2], const void* x, float* const da[2],
+    float* const db[2], void* dx, void* workspace, hipStream_t stream) {
+  if (!ht) return MXS_ERR_ARG;
+  return mxs_nf4_linear_bwd_dx_hp_pair_ws(dy, M, N, K, packed, absmax8, code, absmax2, offset,
+                                          lora_dhp, hp_slices, ldt, lora_at, r, mask, mask_scale,
+                                          lora_dht, ht, x, da, db, dx, workspace, INT64_MAX,
+                                          stream);
 }
 
 // The rotation the grouped forward may apply to its first n_rope problems (attention's q / k).

@@ -115,7 +115,9 @@ def lora_workspace_bytes(M, K, N, r):
 
 
 def projection_workspace_bytes(M, K, N, r=16):
-    """Bytes one workspace needs for every call of a K -> N projection at M tokens."""
+    """Bytes one workspace needs for every call of a K -> N projection at M tokens.  The summed
+    input gradient of two projections (nf4_linear_bwd_dx_hp_pair) runs in it too, on the plan that
+    fits (at few and at many tokens its faster plan takes more: pair_workspace_bytes)."""
     return max(gemm_workspace_bytes(M, N, K), gemm_workspace_bytes(M, K, N),
                lora_workspace_bytes(M, K, N, r) if r else 0)
 
@@ -664,6 +666,21 @@ def bwd_dx_pair_ok(M, N0, N1, K):
     return bool(_lib.lib().mxs_nf4_linear_bwd_dx_pair_ok(M, N0, N1, K))
 
 
+def pair_workspace_bytes(M, N0, N1, K):
+    """Bytes of the summed dX pair's planned workspace."""
+    return int(_lib.lib().mxs_nf4_linear_bwd_dx_pair_workspace_bytes(M, N0, N1, K))
+
+
+def _pair_workspace(M, n0, n1, k, device, ws):
+    """(workspace, its bytes) of the summed dX pair: the plan's own, or the caller's, of at least
+    four fp32 planes [M, K] (the pair then runs on what fits)."""
+    if ws is None:
+        ws = new_workspace(pair_workspace_bytes(M, n0, n1, k), device)
+    else:
+        ws = _workspace(16 * M * k, device, ws)
+    return ws, (0 if ws is None else ws.numel() * ws.element_size())
+
+
 def _dx_pair_operands(dys, packeds, states, lora_dhps, lora_ats, masks):
     """The checked operands of the summed dX pair: (dys, M, N0, N1, K, slices, ldt, r, keep bits,
     device)."""
@@ -703,20 +720,19 @@ def _dx_pair_args(dys, M, n0, n1, k, packeds, states, lora_dhps, S, ldt, lora_at
 def nf4_linear_bwd_dx_hp_pair(dys, packeds, states, lora_dhps, lora_ats, masks=None,
                               mask_scale=1.0, want_t=True, ws=None):
     """(dx, [dht0, dht1]): dX = the sum of nf4_linear_bwd_dx_hp's two input gradients, from ONE
-    split-K launch over both reductions and one reduce (each projection's part is never rounded
-    to fp16 on its own), and each projection's fp16 dHs^T (None unless want_t).  Only where
-    bwd_dx_pair_ok."""
+    launch over both reductions and one reduce (each projection's part is never rounded to fp16
+    on its own), and each projection's fp16 dHs^T (None unless want_t).  Only where
+    bwd_dx_pair_ok.  ws: at least 16 * M * K bytes; pair_workspace_bytes for the planned launch."""
     dys, M, n0, n1, k, S, ldt, r, masks, dev = _dx_pair_operands(dys, packeds, states, lora_dhps,
                                                                  lora_ats, masks)
     dx = torch.empty((M, k), dtype=torch.float16, device=dev)
     dhts = [torch.empty((r, ldt), dtype=torch.float16, device=dev) if want_t else None
             for _ in range(2)]
-    ws = _workspace(int(_lib.lib().mxs_nf4_linear_bwd_dx_pair_workspace_bytes(M, n0, n1, k)),
-                    dev, ws)
-    _lib.call("mxs_nf4_linear_bwd_dx_hp_pair",
+    ws, nbytes = _pair_workspace(M, n0, n1, k, dev, ws)
+    _lib.call("mxs_nf4_linear_bwd_dx_hp_pair_ws",
               *_dx_pair_args(dys, M, n0, n1, k, packeds, states, lora_dhps, S, ldt, lora_ats, r,
                              masks, mask_scale, dhts),
-              _lib.ptr(dx), _lib.ptr(ws), _lib.stream_of(dev))
+              None, None, None, None, _lib.ptr(dx), _lib.ptr(ws), nbytes, _lib.stream_of(dev))
     return dx, dhts
 
 
@@ -735,13 +751,12 @@ def nf4_linear_bwd_dx_hp_pair_grads(dys, packeds, states, lora_dhps, lora_ats, h
     dhts = [torch.empty((r, ldt), dtype=torch.float16, device=dev) for _ in range(2)]
     da = [torch.empty((r, k), dtype=torch.float32, device=dev) for _ in range(2)]
     db = [torch.empty((n, r), dtype=torch.float32, device=dev) for n in (n0, n1)]
-    ws = _workspace(int(_lib.lib().mxs_nf4_linear_bwd_dx_pair_workspace_bytes(M, n0, n1, k)),
-                    dev, ws)
-    _lib.call("mxs_nf4_linear_bwd_dx_hp_pair_grads",
+    ws, nbytes = _pair_workspace(M, n0, n1, k, dev, ws)
+    _lib.call("mxs_nf4_linear_bwd_dx_hp_pair_ws",
               *_dx_pair_args(dys, M, n0, n1, k, packeds, states, lora_dhps, S, ldt, lora_ats, r,
                              masks, mask_scale, dhts),
               _ptr_array([_c(t) for t in hts]), _lib.ptr(x2d), _ptr_array(da), _ptr_array(db),
-              _lib.ptr(dx), _lib.ptr(ws), _lib.stream_of(dev))
+              _lib.ptr(dx), _lib.ptr(ws), nbytes, _lib.stream_of(dev))
     return dx, dhts, list(zip(da, db))
 
 

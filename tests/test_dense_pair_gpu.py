@@ -66,3 +66,32 @@ def test_masks_of_either_projection(cuda, masked, r, widths):
     for (da, db), p, dht, ht, kp in zip(grads, ps, dhts2, hts, keeps):
         da1, db1 = kernels.lora_grads(dht, ht, x, p["dy"], kp, MS)
         assert torch.equal(da, da1) and torch.equal(db, db1)
+
+
+@pytest.mark.parametrize("M", [64, 1430, 3001, 8192])
+def test_callers_workspace(cuda, M):
+    """A workspace of projection_workspace_bytes serves the summed gradient at every token count,
+    whatever the faster plan would take (more fp32 planes at few tokens, the decoded weights at
+    many), and nothing past its end is written; a smaller one than four planes is refused."""
+    from mindxsoup_amd import kernels
+    from mindxsoup_amd.linear4bit import lora_backward_group
+
+    print(f"case dX pair in a caller's workspace M={M}", flush=True)
+    x = torch.randn((M, K), device=cuda).half()
+    ps = [_proj(cuda, 8960, M, 16, 30 + i) for i in range(2)]
+    items = [dict(dy=p["dy"], x2d=x, keep=p["keep"], ht=p["ht"], at=p["a"].t().contiguous(),
+                  bt=p["b"].t().contiguous(), packed=p["packed"], state=p["st"], mask_scale=MS,
+                  s=S, wants=(True, True, True)) for p in ps]
+    nbytes = kernels.projection_workspace_bytes(M, K, 8960)
+    whole = torch.full((nbytes + 4096,), 7, dtype=torch.uint8, device=cuda)
+    got = lora_backward_group(items, ws=whole[:nbytes], sum_dx=True)
+    assert bool((whole[nbytes:] == 7).all())
+    parts = [r[0] for r in lora_backward_group(items)]
+    two = parts[0].float() + parts[1].float()
+    for dx in (got[0][0], lora_backward_group(items, sum_dx=True)[0][0]):
+        assert bool(((dx.float() - two).abs() <= _bound(parts, two)).all())
+    dhps = [kernels.lora_dh_partials(it["dy"], it["bt"], S) for it in items]
+    with pytest.raises(ValueError, match="workspace"):
+        kernels.nf4_linear_bwd_dx_hp_pair([p["dy"] for p in ps], [p["packed"] for p in ps],
+                                          [p["st"] for p in ps], dhps, [it["at"] for it in items],
+                                          ws=whole[:16 * M * K - 4])
