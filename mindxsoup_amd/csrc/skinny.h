@@ -108,6 +108,11 @@ __global__ __launch_bounds__(64 * (kSkinnyWaves + 1)) void k_nf4_skinny(SkinnyGr
         }
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf, wf, acc, 0, 0, 0);
       }
+      if (n0 == 0 && a.lora_hp && a.lora_ht) {  // a row length past the 16 rows: zeros
+        const int pad = a.ldt - kSkinnyRows;
+        for (int i = lane; i < a.r * pad; i += 64)
+          a.lora_ht[(int64_t)(i / pad) * a.ldt + kSkinnyRows + i % pad] = (_Float16)0.0f;
+      }
     }
   }
   // acc[v] = C[4 g + v][n0 + c16]; waves past nw have none

@@ -18,8 +18,9 @@ def _close(got, want):
     assert bool((d <= bound).all()), (d - bound).max().item()
 
 
-# M: the 16-row block's edges; N: a partial 16-column group never occurs (N % 64 == 0); K: shorter
-# than one 128-wide chunk, a half chunk at the end, more chunks than one batch per wave
+# M: the 16-row block's edges; N: whole 16-column groups (partial ones, which only the C ABI takes:
+# test_few_tokens_abi_gpu.py); K: shorter than one 128-wide chunk, a half chunk at the end, more
+# chunks than one batch per wave
 @pytest.mark.parametrize("M", [1, 5, 16, 17])
 @pytest.mark.parametrize("n,k,r", [(64, 64, 16), (1536, 1536, 16), (256, 1472, 32),
                                    (1536, 8960, 16), (192, 320, 128)])
