@@ -122,9 +122,10 @@ int mxs_nf4_linear_fwd(const void* x, int M, int K, int N, const void* packed,
  * memory: code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.
  * No counterpart in the reference (its forward allocates through torch).  Nothing is allocated:
  * split-K partials go to a file-scope device array of MXS_NF4_SCRATCH_BYTES, whose address is
- * looked up once per device on the first call made with that device current.  That lookup is
- * not a stream operation: under HIP graph capture, make one call on the device before the
- * capture begins; the calls after it launch kernels only and are capturable.  A plan needing
+ * looked up once per device on the first call made with that device current, whatever its plan.
+ * That lookup is not a stream operation: under HIP graph capture, make one call on the device
+ * before the capture begins; the calls after it launch kernels only and are capturable.  (A first
+ * call on a capturing stream looks nothing up where its plan needs no partials.)  A plan needing
  * more (splits * M * N * 4 bytes) returns MXS_ERR_SIZE with nothing launched.  Every call on
  * one GPU shares that array: calls that overlap in time on one GPU (other streams or threads)
  * race and must be serialized by the caller.  Same results as mxs_nf4_linear_fwd, with the bits

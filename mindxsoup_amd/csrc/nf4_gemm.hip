@@ -3401,6 +3401,20 @@ static int scratch_address(void** out) {
   return MXS_OK;
 }
 
+// The lookup made ahead of need: any call outside a capture does it, so that a later captured one
+// finds the address whatever plan the first had.  A capturing stream is left alone.
+static void scratch_lookup_ahead(hipStream_t stream) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices ||
+      g_scratch[dev].load(std::memory_order_acquire))
+    return;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusActive;
+  void* p = nullptr;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) (void)hipGetLastError();
+  else if (status == hipStreamCaptureStatusNone && scratch_address(&p) != MXS_OK)
+    (void)hipGetLastError();
+}
+
 // The two problems of the summed dX pair (mxs_nf4_linear_bwd_dx_hp_pair's checks): MXS_OK,
 // 1 when there is nothing to compute, or an error code.
 static int dx_pair_args(const void* const dy[2], int M, const int N[2], int K,
@@ -4128,6 +4142,7 @@ extern "C" int mxs_nf4_linear_fwd_noalloc(const void* x, int M, int K, int N, co
                                           const void* lora_b, int r, void* y, int cfg,
                                           int splits, hipStream_t stream) {
   if (M < 0 || K < 0 || N < 0) return MXS_ERR_ARG;
+  scratch_lookup_ahead(stream);
   if (cfg < 0 && skinny_takes(M, N, K))
     return mxs_nf4_linear_fwd(x, M, K, N, packed, absmax8, code, absmax2, offset, bias, lora_h,
                               lora_b, r, y, nullptr, -1, 1, stream);
