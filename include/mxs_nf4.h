@@ -422,11 +422,13 @@ int mxs_silu_mul_bwd(const void* grad, void* gate, void* up, int64_t n, hipStrea
  * solution/attention.py:259-266): problem i has x[i] [M, K], out_features N[i], its NF4 weight
  * (packed[i] .. offset[i]), bias[i], LoRA partials lora_hp[i] (hp_slices, ldt, r shared),
  * lora_b[i] [N[i], r], lora_ht[i], output y[i] [M, N[i]]; the bias, lora_hp, lora_b and lora_ht
- * arrays may be NULL (or any entry: no bias / no LoRA term).  Every problem runs unsplit on
- * warp-specialized tiles with 8 producer waves, 128x64 when all the problems' tiles fit the CUs
- * in one round (q, k and v at 1024 tokens), else 128x128: the same bits as mxs_nf4_linear_fwd_hp
- * with one split for each (every warp-specialized configuration accumulates in one order; the
- * N = 256 projections alone would plan split-K tiles and a reduce). */
+ * arrays may be NULL (or any entry: no bias / no LoRA term).  Up to 16 tokens every problem runs
+ * on the few-token kernel: the bits of mxs_nf4_linear_fwd_hp (cfg -1) for each.  Past that every
+ * problem runs unsplit on warp-specialized tiles with 8 producer waves, 128x64 when all the
+ * problems' tiles fit the CUs in one round (q, k and v at 1024 tokens), else 128x128: the same
+ * bits as mxs_nf4_linear_fwd_hp on those tiles with one split for each (cfg 6 to 12, splits 1:
+ * every warp-specialized configuration accumulates in one order; alone a projection may plan
+ * split-K tiles and a reduce, as the N = 256 ones do). */
 int mxs_nf4_linear_fwd_hp_group(int n, const void* const x[], int M, int K, const int N[],
                                 const void* const packed[], const void* const absmax8[],
                                 const float* const code[], const float* const absmax2[],
@@ -441,9 +443,9 @@ int mxs_nf4_linear_fwd_hp_group(int n, const void* const x[], int M, int K, cons
  * for i < n_rope holds rot(the fp16 projection output), each 128-column head rotated by the
  * fp32 cos / sin row of its token (row m is token m % n_tokens of sequence m / n_tokens; rows
  * at b * cos_stride_b + t * cos_stride_t, cos_stride_b may be 0; 16-byte aligned, strides
- * multiples of 4).  The stored fp16 has the bits of mxs_nf4_linear_fwd_hp_group followed by
- * mxs_qkv_rope (forward, no LoRA term) on those outputs; the remaining outputs (v) are
- * unchanged.  N[i] of a rotated output: a multiple of 128; M a multiple of n_tokens. */
+ * multiples of 4).  At every token count the stored fp16 has the bits of
+ * mxs_nf4_linear_fwd_hp_group followed by mxs_qkv_rope (forward, no LoRA term) on those outputs;
+ * the remaining outputs (v) are unchanged.  N[i] of a rotated output: a multiple of 128; M a multiple of n_tokens. */
 int mxs_nf4_linear_fwd_hp_group_rope(int n, const void* const x[], int M, int K, const int N[],
                                      const void* const packed[], const void* const absmax8[],
                                      const float* const code[], const float* const absmax2[],

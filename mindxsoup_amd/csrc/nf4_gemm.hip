@@ -3986,7 +3986,7 @@ static int fwd_hp_group(int n, const void* const x[], int M, int K, const int N[
     probs[live++] = a;
   }
   if (live == 0) return MXS_OK;
-  if (rs.n_rope == 0 && skinny_takes(M, 1, K)) return launch_skinny(probs, live, stream);
+  if (skinny_takes(M, 1, K)) return launch_skinny(probs, live, stream);
   DensePlan d;
   if (workspace && live == n && dense_group_plan(n, M, N, K, rs.n_rope > 0, &d))
     return launch_dense(false, probs, n, false, d, workspace, true, nullptr, stream);

@@ -24,9 +24,27 @@ struct SkinnyGroup {
   int n;
 };
 
-// Lane l holds column n0 + l % 16 of the weight and row l % 16 of x, lane
-// group g = l / 16 the 32 reduction indices 32 g of its chunk; multiply j takes 8 j .. 8 j + 7 of
-// them on both sides.
+// The rotated output of row m, column col (column c of the workgroup): the lane 8 away in c holds
+// the value 64 columns away in the head.  Every lane of the wave calls it.
+__device__ __forceinline__ float skinny_rotate(const GemmArgs& a, float sum, int m, int c,
+                                               int col) {
+#pragma clang fp contract(off)
+  const float x = (float)(_Float16)sum, other = __shfl_xor(x, 8, 64);
+  if (m >= a.M) return x;
+  const int b = m / a.rope_T, t = m - b * a.rope_T;
+  const int64_t at = (int64_t)b * a.rope_cs_b + (int64_t)t * a.rope_cs_t + (col & 127);
+  const float s = a.rope_sin[at];
+  return x * a.rope_cos[at] + other * (c & 8 ? s : -s);
+}
+
+// Lane l holds column l % 16 of the workgroup's 16 and row l % 16 of x, lane group g = l / 16 the
+// 32 reduction indices 32 g of its chunk; multiply j takes 8 j .. 8 j + 7 of them on both sides.
+// The workgroup's columns are 16 neighbours, or, where the output is rotated, 8 of a head's first
+// half and the 8 they pair with 64 further on, so that a rotation's two values meet in one wave:
+// rope_rotate's arithmetic on the fp16 values, a group then having the bits of the same group
+// followed by the rotation launch (q, k and v of 1 token: 5.3 us rotated, 4.7 not; rotated on the
+// tile kernels 12.7).  ROPE: some problem of the launch is rotated.
+template <bool ROPE>
 __global__ __launch_bounds__(64 * (kSkinnyWaves + 1)) void k_nf4_skinny(SkinnyGroup grp) {
   __shared__ float s_nf4[16];
   __shared__ float s_code[256];
@@ -40,7 +58,12 @@ __global__ __launch_bounds__(64 * (kSkinnyWaves + 1)) void k_nf4_skinny(SkinnyGr
   const int lw = ((int)blockDim.x >> 6) - 1;  // the wave of bias and LoRA
   const int c16 = lane & 15, g = lane >> 4;
   const int n0 = ((int)blockIdx.x - grp.start[pi]) * 16;
-  const int n = min(n0 + c16, a.Nc - 1);
+  const bool rot = ROPE && a.rope_cos;
+  // output column of the workgroup's column c
+  auto column = [&](int c) {
+    return rot ? (n0 & ~127) + ((n0 & 127) >> 1) + (c & 7) + ((c & 8) << 3) : n0 + c;
+  };
+  const int n = min(column(c16), a.Nc - 1);
   const int chunks = (a.Kr + kSkinnyChunk - 1) / kSkinnyChunk;
   const float off = a.offset[0];
   const int64_t row = (int64_t)n * a.Kr;
@@ -121,11 +144,14 @@ __global__ __launch_bounds__(64 * (kSkinnyWaves + 1)) void k_nf4_skinny(SkinnyGr
     for (int v = 0; v < 4; v++) red[wave][4 * g + v][c16] = acc[v];
   __syncthreads();
   for (int i = t; i < 256; i += (int)blockDim.x) {
-    const int m = i >> 4, c = i & 15;
-    if (m >= a.M || n0 + c >= a.Nc) continue;
+    const int m = i >> 4, c = i & 15, col = column(c);
     float sum = red[lw][m][c];  // bias and LoRA first, as the tile kernels' accumulators start
     for (int v = 0; v < nw; v++) sum += red[v][m][c];
-    a.C[(int64_t)m * a.ldc + n0 + c] = (_Float16)sum;
+    if constexpr (ROPE) {
+      if (rot) sum = skinny_rotate(a, sum, m, c, col);
+    }
+    if (m >= a.M || col >= a.Nc) continue;
+    a.C[(int64_t)m * a.ldc + col] = (_Float16)sum;
   }
 }
 
@@ -146,8 +172,10 @@ static int launch_skinny(const GemmArgs* probs, int n, hipStream_t stream) {
   g.n = n;
   int64_t total = 0;
   int nw = 1;
+  bool rope = false;
   for (int i = 0; i < n; i++) {
     g.p[i] = probs[i];
+    rope = rope || probs[i].rope_cos;
     g.start[i] = (int)total;
     total += (probs[i].Nc + 15) / 16;
     g.nw[i] = skinny_waves(probs[i].Nc, probs[i].Kr);
@@ -155,7 +183,9 @@ static int launch_skinny(const GemmArgs* probs, int n, hipStream_t stream) {
   }
   if (total > 0x7fffffff) return MXS_ERR_SIZE;
   g.start[n] = (int)total;
-  hipLaunchKernelGGL(k_nf4_skinny, dim3((unsigned)total), dim3(64 * (nw + 1)), 0, stream, g);
+  const dim3 grid((unsigned)total), block(64 * (nw + 1));
+  if (rope) hipLaunchKernelGGL(k_nf4_skinny<true>, grid, block, 0, stream, g);
+  else hipLaunchKernelGGL(k_nf4_skinny<false>, grid, block, 0, stream, g);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? MXS_OK : (int)e;
 }
