@@ -257,10 +257,11 @@ int mxs_nf4_linear_bwd_dx_hp_pair_ws(
  * entry); the two share M, K, r, ldt and hp_slices.  Their tiles share the GPU's rounds: at
  * 1024 tokens 2 x 224 tiles of 256 x 160 would take 1.75 rounds of 256 CUs, so where it fills
  * the CUs better the launch cuts the columns into 256 x 160 tiles and narrower 256 x 128 ones
- * (at 1024 tokens: 192 + 320 tiles, each CU running one of each or two narrow ones).  Only
- * where mxs_nf4_linear_fwd_pair_ok(M,
- * N[0], N[1], K) is 1 (both plan the unsplit 256 x 160 kernel: N[0] == N[1] >= 4096), else
- * MXS_ERR_SIZE. */
+ * (at 1024 tokens: 192 + 320 tiles, each CU running one of each or two narrow ones); up to 16
+ * tokens both run on the few-token kernel.  Takes N[0] == N[1] >= 4096 at every token count, else
+ * MXS_ERR_SIZE.  Where mxs_nf4_linear_fwd_pair_ok(M, N[0], N[1], K) is 0 for such outputs (K >= N:
+ * each alone would split its long reduction), the pair still runs both unsplit, which is slower
+ * than the two calls and adds in another order. */
 int mxs_nf4_linear_fwd_hp_pair(const void* x, int M, int K, const int N[2],
                                const void* const packed[2], const void* const absmax8[2],
                                const float* const code[2], const float* const absmax2[2],
@@ -269,8 +270,8 @@ int mxs_nf4_linear_fwd_hp_pair(const void* x, int M, int K, const int N[2],
                                const void* const lora_b[2], int r, void* const lora_ht[2],
                                void* const y[2], hipStream_t stream);
 
-/* 1 when mxs_nf4_linear_fwd_hp_pair takes two projections [K -> N0] and [K -> N1] at M tokens,
- * else 0. */
+/* 1 when mxs_nf4_linear_fwd_hp_pair takes two projections [K -> N0] and [K -> N1] at M tokens and
+ * gives the bits of two mxs_nf4_linear_fwd_hp calls (cfg -1 with their workspace), else 0. */
 int mxs_nf4_linear_fwd_pair_ok(int M, int N0, int N1, int K);
 
 /* 1 when mxs_nf4_linear_bwd_dx_hp_pair takes two projections [K -> N0] and [K -> N1] at M

@@ -2361,8 +2361,9 @@ static double few_us(int cus, int cfg, int sp, int M, int Nc, int steps) {
 // Measured, planned / base: gate forward 12.8 / 24.9 us at 64 tokens, 18.6 / 25.4 at 200, 20.1 /
 // 26.1 at 300, 28.1 / 32.8 at 700; down forward 15.0 / 27.4, 20.5 / 31.7, 24.8 / 33.0; a
 // 4096 x 11008 projection (wide and long: one split in the base plan) 24.6 / 57.3, 36.8 / 62.6,
-// 54.1 / 76.9.  A wide output's 24-step reduction stays whole, so that gate's and up's launches
-// of any kind keep one order of sums, and so does every short reduction of the input gradient.
+// 54.1 / 76.9.  An output wider than 4096 and than its reduction (gate, up) keeps that whole, so
+// that one projection and both in one launch add in one order, and so does every short reduction
+// of the input gradient.
 static void choose(int M, int Nc, int Kr, bool bwd, int* cfg, int* splits) {
   choose_base(M, Nc, Kr, bwd, cfg, splits);
   const int cus = cu_count();
@@ -2374,7 +2375,7 @@ static void choose(int M, int Nc, int Kr, bool bwd, int* cfg, int* splits) {
     for (int c : {12, 10, bwd ? 11 : 9, 6, 7})
       for (int sp = 1; sp <= 8; sp++) {
         if (sp > 1 &&
-            (steps / sp < 6 || !(Kr >= 4096 || (!bwd && Nc < 4096)) ||
+            (steps / sp < 6 || !(bwd ? Kr >= 4096 : Nc < 4096 || Kr >= Nc) ||
              (sp > base_sp && (int64_t)sp * M * Nc * 4 > (int64_t)MXS_NF4_SCRATCH_BYTES)))
           break;
         if (ceil_div(steps, ceil_div(steps, sp)) != sp) continue;
@@ -3074,13 +3075,24 @@ static int launch_ws_fwd_pair_mixed(const GemmArgs& a0, const GemmArgs& a1, int 
   return e == hipSuccess ? MXS_OK : (int)e;
 }
 
-// The forward pair takes two problems [K -> N] that each plan the unsplit 256x160 kernel.
-static bool fwd_pair_plan_ok(int M, int N0, int N1, int K) {
+// The forward pair takes two problems [K -> N] whose base plan is the unsplit 256x160 kernel.
+static bool fwd_pair_takes(int M, int N0, int N1, int K) {
   if (M <= 0 || N0 != N1 || K <= 0 || K % kBK) return false;
   int c, sp;
   choose_base(M, N0, K, false, &c, &sp);
   return c == 7 && sp == 1 && (int64_t)N0 * K < (int64_t(1) << 32) &&
          (int64_t)256 * K * 2 < (int64_t(1) << 32);
+}
+
+// The pair has the bits of two launches: each alone would run unsplit too.
+static bool fwd_pair_plan_ok(int M, int N0, int N1, int K) {
+  if (!fwd_pair_takes(M, N0, N1, K)) return false;
+  if (skinny_takes(M, N0, K)) return true;
+  DensePlan d;
+  if (dense_takes(M, N0, K) && dense_plan(M, N0, K, false, false, &d)) return d.splits <= 1;
+  int c, sp;
+  choose(M, N0, K, false, &c, &sp);
+  return sp <= 1;
 }
 
 // Splits of each of the pair's reductions (256x96 tiles, two problems): two, so that a workgroup
@@ -3781,7 +3793,7 @@ int mxs_nf4_linear_fwd_hp_pair(const void* x, int M, int K, const int N[2],
       !lora_b || !y)
     return MXS_ERR_ARG;
   if (M == 0) return MXS_OK;
-  if (!fwd_pair_plan_ok(M, N[0], N[1], K)) return MXS_ERR_SIZE;
+  if (!fwd_pair_takes(M, N[0], N[1], K)) return MXS_ERR_SIZE;
   GemmArgs p[2];
   for (int i = 0; i < 2; i++) {
     GemmArgs a{};

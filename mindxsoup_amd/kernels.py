@@ -609,19 +609,22 @@ def nf4_linear_bwd_dx_hp(dy2d, packed, state, lora_dhp, lora_at, mask=None, mask
 
 
 def fwd_pair_ok(M, N0, N1, K):
-    """Whether nf4_linear_fwd_hp_pair takes two projections [K -> N0], [K -> N1] at M tokens."""
+    """Whether nf4_linear_fwd_hp_pair runs two projections [K -> N0], [K -> N1] at M tokens in one
+    launch with the bits of two."""
     return bool(_lib.lib().mxs_nf4_linear_fwd_pair_ok(M, N0, N1, K))
 
 
 def nf4_linear_fwd_hp_pair(x2d, packeds, states, lora_hps, lora_bs, biases=None):
     """nf4_linear_fwd_hp for two projections over the same x2d in one launch (grid z selects the
-    projection; the same bits as two calls): [(y, ht), (y, ht)].  Only where fwd_pair_ok."""
+    projection; the same bits as two calls): [(y, ht), (y, ht)].  Only for equal outputs of at
+    least 4096; where each alone would split its reduction (fwd_pair_ok is False), two calls."""
     (n0, k), (n1, k1) = states[0].shape, states[1].shape
     if x2d.dtype != torch.float16 or x2d.dim() != 2 or x2d.shape[1] != k or k1 != k:
         raise ValueError("x must be fp16 [M, in_features] of two weights [N_i, K]")
     x2d = x2d.contiguous()
     M = x2d.shape[0]
-    if not fwd_pair_ok(M, n0, n1, k):
+    one_launch = fwd_pair_ok(M, n0, n1, k)
+    if not one_launch and (M == 0 or n0 != n1 or n0 < 4096 or n0 * k >= 2 ** 32):
         raise ValueError(f"the forward pair does not take [{k} -> {n0}], [{k} -> {n1}] at {M} "
                          "tokens")
     S, ldt, r = lora_hps[0].shape
@@ -631,6 +634,9 @@ def nf4_linear_fwd_hp_pair(x2d, packeds, states, lora_hps, lora_bs, biases=None)
             raise ValueError("lora_hp [slices, ldt, r] fp32 (one shape) and lora_b [N, r]")
     biases = biases or [None, None]
     biases = [None if b is None else b.to(torch.float16).contiguous() for b in biases]
+    if not one_launch:
+        return [nf4_linear_fwd_hp(x2d, pk, st, hp, b, bias)
+                for pk, st, hp, b, bias in zip(packeds, states, lora_hps, lora_bs, biases)]
     dev = x2d.device
     for pk, st in zip(packeds, states):
         check_nf4_operands(pk, st, dev)

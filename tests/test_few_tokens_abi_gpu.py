@@ -52,3 +52,31 @@ def test_partial_column_groups(cuda, M, n, k):
     want = kernels.nf4_linear_fwd(x, packed, st, bias, cfg=10, splits=1).float()
     bound = 2.0 ** -10 * want.abs() + 2.0 ** -20 * want.abs().max()
     assert bool(((got.float() - want).abs() <= bound).all())
+
+
+# gate / up widths (N > K), where one projection alone must not split what the pair sums whole; and
+# long reductions (K >= N), where it does split and the pair runs as two launches
+@pytest.mark.parametrize("M,n,k", [(17, 11008, 4096), (64, 11008, 4096), (200, 11008, 4096),
+                                   (200, 14336, 4096), (64, 4096, 4096), (1024, 4096, 4096),
+                                   (40, 4096, 14336), (40, 8960, 1536)])
+def test_forward_pair_has_the_bits_of_single_launches(cuda, M, n, k):
+    from mindxsoup_amd import kernels, ops
+
+    print(f"case forward pair M={M} n={n} k={k}", flush=True)
+    g, p0, s0 = _weight(cuda, n, k, 1)
+    _, p1, s1 = _weight(cuda, n, k, 2)
+    rnd = lambda *s: torch.randn(s, device=cuda, generator=g)  # noqa: E731
+    x, bias = rnd(M, k).half(), rnd(n).half()
+    As = [(rnd(16, k) / k ** 0.5).half() for _ in range(2)]
+    Bs = [(rnd(n, 16) * 0.1).half() for _ in range(2)]
+    rows = kernels.lora_h_partials_group([x, x], As, 2.0, None, 1.0, Bs)
+    hps = [o[0] for o in rows]
+    assert kernels.fwd_pair_ok(M, n, n, k) == (n > k)
+    pair = kernels.nf4_linear_fwd_hp_pair(x, [p0, p1], [s0, s1], hps, Bs, [bias, None])
+    both = ops.load().lora_fwd_group(
+        x, As, Bs, *map(list, zip(ops.nf4(p0, s0), ops.nf4(p1, s1))), [bias, None], [None, None],
+        1.0, 2.0, False, None, None, 0)
+    for i, (p, s, b) in enumerate(((p0, s0, bias), (p1, s1, None))):
+        y, ht = kernels.nf4_linear_fwd_hp(x, p, s, hps[i], Bs[i], b)
+        assert torch.equal(pair[i][0], y) and torch.equal(pair[i][1], ht)
+        assert torch.equal(both[0][i], y) and torch.equal(both[1][i], ht)
