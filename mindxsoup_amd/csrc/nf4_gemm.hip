@@ -2665,10 +2665,25 @@ static bool skinny_takes(int M, int Nc, int Kr) {
   return M >= 1 && M <= kSkinnyRows && Nc > 0 && Kr > 0 && Kr % kBK == 0;
 }
 
+// The planned kernel for a GEMM [M, Nc] over Kr takes the SwiGLU output: a warp-specialized
+// configuration that none of its fallback conditions sends to the all-wave kernel.
+static bool glu_plan_ok(int M, int Nc, int Kr, bool bwd) {
+  if (M <= 0 || Nc <= 0 || Kr <= 0 || Nc % 8 != 0 || Kr % kBK != 0) return false;
+  int cfg, sp;
+  choose(M, Nc, Kr, bwd, &cfg, &sp);
+  if (cfg < 6 || cfg >= kNumCfg) return false;
+  static const int kPW[] = {4, 4, 4, 4, 8, 8, 8};
+  const int bm = kWsBM[cfg - 6], pw = kPW[cfg - 6];
+  return (int64_t)Nc * Kr < (int64_t(1) << 32) && (int64_t)bm * Kr * 2 < (int64_t(1) << 32) &&
+         !(bwd && Nc < (pw == 8 ? 16 : 32));
+}
+
 static int gemm_entry(bool bwd, const GemmArgs& a, int cfg, int splits, hipStream_t stream) {
   const int c = check_gemm(bwd, a);
   if (c != MXS_OK) return c == 1 ? MXS_OK : c;
   if (cfg < 0) {
+    // the SwiGLU forward is taken and refused by the plan's rule at every token count
+    if (a.glu == 1 && !glu_plan_ok(a.M, a.Nc, a.Kr, false)) return MXS_ERR_SIZE;
     if (!bwd && skinny_takes(a.M, a.Nc, a.Kr)) {
       const int rc = launch_skinny(&a, 1, stream);
       if (rc != MXS_OK || a.glu != 1) return rc;
@@ -2729,19 +2744,6 @@ static bool grads_fusable(int M, int N, int K, int r, int* cfg_out, int* nw_out)
   *cfg_out = cfg;
   *nw_out = nw;
   return true;
-}
-
-// The planned kernel for a GEMM [M, Nc] over Kr takes the SwiGLU output: a warp-specialized
-// configuration that none of its fallback conditions sends to the all-wave kernel.
-static bool glu_plan_ok(int M, int Nc, int Kr, bool bwd) {
-  if (M <= 0 || Nc <= 0 || Kr <= 0 || Nc % 8 != 0 || Kr % kBK != 0) return false;
-  int cfg, sp;
-  choose(M, Nc, Kr, bwd, &cfg, &sp);
-  if (cfg < 6 || cfg >= kNumCfg) return false;
-  static const int kPW[] = {4, 4, 4, 4, 8, 8, 8};
-  const int bm = kWsBM[cfg - 6], pw = kPW[cfg - 6];
-  return (int64_t)Nc * Kr < (int64_t(1) << 32) && (int64_t)bm * Kr * 2 < (int64_t(1) << 32) &&
-         !(bwd && Nc < (pw == 8 ? 16 : 32));
 }
 
 // The GEMMs of several problems in one launch of one warp-specialized tile configuration with 8

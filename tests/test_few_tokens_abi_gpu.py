@@ -80,3 +80,17 @@ def test_forward_pair_has_the_bits_of_single_launches(cuda, M, n, k):
         y, ht = kernels.nf4_linear_fwd_hp(x, p, s, hps[i], Bs[i], b)
         assert torch.equal(pair[i][0], y) and torch.equal(pair[i][1], ht)
         assert torch.equal(both[0][i], y) and torch.equal(both[1][i], ht)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17])
+def test_swiglu_forward_refused_where_it_was(cuda, M):
+    """A width whose plan has no SwiGLU epilogue is refused at few tokens too, nothing written."""
+    from mindxsoup_amd import kernels
+
+    n, k = 256, 1536
+    print(f"case glu refused M={M}", flush=True)
+    _, packed, st = _weight(cuda, n, k, 3)
+    assert not kernels.glu_fused(M, n, k, False)
+    x, gate = (torch.randn((M, w), device=cuda).half() for w in (k, n))
+    with pytest.raises(RuntimeError, match="shape outside"):
+        kernels.nf4_linear_fwd_glu(x, packed, st, gate)
