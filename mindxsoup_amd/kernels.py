@@ -46,16 +46,23 @@ def keep_bits(mask, M, K):
     word k / 32 of row m set where element (m, k) is kept.  A byte mask [M, K] (uint8, int8 or
     bool; nonzero = kept, the reference's int8 `keep`, solution/dropout.py:64) is packed by one
     launch (mxs_keep_pack); a mask already in bits passes through; None stays None."""
-    if mask is None:
+    if check_keep(mask, M, K) is None:
         return None
-    kw = keep_words(K)
-    if mask.dtype == torch.int32 and tuple(mask.shape) == (M, kw):
+    if mask.dtype == torch.int32:
         return mask.contiguous()
-    if mask.dtype in (torch.uint8, torch.int8, torch.bool) and tuple(mask.shape) == (M, K):
-        src = mask.contiguous().view(torch.uint8)
-        bits = torch.empty((M, kw), dtype=torch.int32, device=mask.device)
-        _lib.call("mxs_keep_pack", _lib.ptr(src), M, K, _lib.ptr(bits), _lib.stream_of(mask.device))
-        return bits
+    src = mask.contiguous().view(torch.uint8)
+    bits = torch.empty((M, keep_words(K)), dtype=torch.int32, device=mask.device)
+    _lib.call("mxs_keep_pack", _lib.ptr(src), M, K, _lib.ptr(bits), _lib.stream_of(mask.device))
+    return bits
+
+
+def check_keep(mask, M, K):
+    """The mask, None or one that keep_bits takes; ValueError for any other."""
+    kw = keep_words(K)
+    if mask is None or (mask.dtype == torch.int32 and tuple(mask.shape) == (M, kw)) or \
+            (mask.dtype in (torch.uint8, torch.int8, torch.bool)
+             and tuple(mask.shape) == (M, K)):
+        return mask
     raise ValueError(f"mask must be a uint8 [{M}, {K}] keep mask or int32 [{M}, {kw}] keep bits, "
                      f"got {mask.dtype} {tuple(mask.shape)}")
 

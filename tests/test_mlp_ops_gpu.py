@@ -70,3 +70,22 @@ def test_unequal_scalings_pack_masks_once(cuda, monkeypatch):
     y = mlp(x)
     y.backward(torch.randn_like(y))
     assert packed == [(37, 1536), (37, 1536), (37, 2048)]
+
+
+@pytest.mark.parametrize("name", ["gate_proj", "down_proj"])
+def test_wrong_keep_mask_is_a_value_error(cuda, monkeypatch, name):
+    """A caller's keep mask of another shape or dtype is refused with one error on both paths,
+    before anything is launched."""
+    from mindxsoup_amd import ops
+
+    print(f"case mlp wrong keep {name}", flush=True)
+    mlp = _mlp(cuda, 1536, 2048, 16, 0.05).train()
+    x = torch.randn((1, 37, 1536), device=cuda, requires_grad=True)
+    width = getattr(mlp, name).base_layer.in_features
+    for enabled in (True, False):
+        monkeypatch.setattr(ops, "ENABLED", enabled)
+        for keep in (torch.ones((37, width - 1), dtype=torch.uint8, device=cuda),
+                     torch.ones((37, width), dtype=torch.int64, device=cuda)):
+            getattr(mlp, name).next_keep = keep
+            with pytest.raises(ValueError, match="keep mask"):
+                mlp(x)
