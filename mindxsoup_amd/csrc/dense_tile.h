@@ -281,7 +281,9 @@ __device__ __forceinline__ void rope_rotate_head(const GemmArgs& a, float16_t (&
 // 32-deep K-steps, so that one's ends hide behind the other's multiplies (1.5 times the copies:
 // 280 against 220 us).
 // NSUM > 1: up to NSUM problems with one output, their reductions one after the other into the
-// same accumulators (GemmArgs as[0..nsum)).
+// same accumulators (GemmArgs as[0..nsum)).  Every problem has keep bits or none does: with the
+// test per problem the compiler spilled inside the K loop (gate and up's dX at 8192 tokens: 1099 us
+// instead of 506), so the host keeps mixed masks on the fused kernel.
 template <int BN, bool BWD, bool GLU, int NSUM, bool ROPE>
 __device__ __forceinline__ void dense_tile(const GemmArgs* as, int nsum, int bx, int by) {
   constexpr int BM = kDenseBM, TM = 2, TN = BN / 64, NT = kDenseNT;
@@ -334,6 +336,7 @@ __device__ __forceinline__ void dense_tile(const GemmArgs* as, int nsum, int bx,
   // accumulator start: bias and the LoRA term (first split), its operands staged in stage 1
   const bool lora = (int)blockIdx.z == a.zf && (a.lora_hp || a.lora_h);
   const bool lora16 = lora && a.r == 16;
+  const bool kmask = BWD && lora && a.mask;
   using MS = MaskStage<BM, BN, NT>;
   constexpr int LSH = (BM + BN) * 16;
   static_assert(LSH * 2 + BM * MS::KST <= (int)STAGE, "staged operands fit a stage");
@@ -342,9 +345,6 @@ __device__ __forceinline__ void dense_tile(const GemmArgs* as, int nsum, int bx,
   float16_t acc[TM][TN];
   AccStart<TM, TN, BWD> start;
   auto begin = [&](const GemmArgs& p, float16_t (&c)[TM][TN]) {
-    // of summed problems any may have keep bits and any none; uniform over the workgroup, so its
-    // waves meet at the same barriers
-    const bool kmask = BWD && lora && p.mask;
     if (lora16 || kmask) {
       LoraStage<BM, BN, NT> lst;
       MS mst;

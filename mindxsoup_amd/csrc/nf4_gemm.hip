@@ -2609,6 +2609,10 @@ static int launch_dense(bool bwd, const GemmArgs* probs, int n, bool sum, const 
   int steps = 0;
   int64_t tiles = 0;
   bool rope = false;
+  for (int i = 1; sum && i < n; i++)  // what the kernel takes from problem 0 for all
+    if (!probs[i].mask != !probs[0].mask || !probs[i].lora_hp != !probs[0].lora_hp ||
+        !probs[i].lora_h != !probs[0].lora_h || probs[i].r != probs[0].r)
+      return MXS_ERR_ARG;
   for (int i = 0; i < n; i++) {
     GemmArgs a = probs[i];
     a.w16 = reinterpret_cast<const _Float16*>(w);
@@ -3184,8 +3188,9 @@ static bool dense_pair_plan(int M, const int N[2], int K, DensePlan* d) {
 }
 
 // The pair's plan within a caller's workspace: decoded weights where planned and the bytes (and
-// their alignment) are there, else the fused launch with its planned splits, else with two (four
-// planes, the least any caller brings).
+// their alignment) are there and both problems have keep bits or neither (the dense kernel's
+// condition), else the fused launch with its planned splits, else with two (four planes, the least
+// any caller brings).
 struct PairPlan {
   bool dense;
   DensePlan d;
@@ -3196,8 +3201,9 @@ static int64_t pair_planes_bytes(int M, int K, int splits) {
   return (int64_t)2 * splits * M * K * (int64_t)sizeof(float);
 }
 
-static bool pair_plan(int M, const int N[2], int K, const void* ws, int64_t bytes, PairPlan* p) {
-  p->dense = dense_pair_plan(M, N, K, &p->d) && (uintptr_t)ws % 16 == 0 &&
+static bool pair_plan(int M, const int N[2], int K, bool mixed_masks, const void* ws,
+                      int64_t bytes, PairPlan* p) {
+  p->dense = !mixed_masks && dense_pair_plan(M, N, K, &p->d) && (uintptr_t)ws % 16 == 0 &&
              dense_sum_bytes(2, M, N, K, p->d) <= bytes;
   p->splits = pair_splits(M, N, K);
   if (pair_planes_bytes(M, K, p->splits) > bytes) p->splits = 2;
@@ -3869,7 +3875,8 @@ int mxs_nf4_linear_bwd_dx_hp_pair_ws(
   }
   if (c != MXS_OK) return c;
   PairPlan plan;
-  if (!pair_plan(M, N, K, workspace, workspace_bytes, &plan)) return MXS_ERR_SIZE;
+  const bool mixed_masks = (p[0].mask != nullptr) != (p[1].mask != nullptr);
+  if (!pair_plan(M, N, K, mixed_masks, workspace, workspace_bytes, &plan)) return MXS_ERR_SIZE;
   if (!grads)
     return plan.dense
         ? launch_dense(true, p, 2, true, plan.d, workspace, true, nullptr, stream)

@@ -1,6 +1,6 @@
-"""The summed input gradient of gate and up from decoded weights (k_dense_gemm over two reductions,
-mxs_nf4_linear_bwd_dx_hp_pair at many tokens): each projection's own keep mask or none, ranks
-staged through LDS (16) and read from memory, unequal widths.
+"""The summed input gradient of gate and up at many tokens (mxs_nf4_linear_bwd_dx_hp_pair): from
+decoded weights (k_dense_gemm over two reductions) with a keep mask on both or on neither, on the
+fused kernel with a mask on one; ranks staged through LDS (16) and read from memory, unequal widths.
 
 Reference: the two projections' single input gradients on the fused kernels, each rounded to fp16,
 added in fp32.  The summed launch rounds once, so the two differ by the parts' roundings (half an
