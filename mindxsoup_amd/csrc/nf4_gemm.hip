@@ -2540,11 +2540,19 @@ constexpr int kDenseTokens = 769;
 static bool dense_plan(int M, int Nc, int Kr, bool bwd, bool glu, DensePlan* d) {
   const int cus = cu_count();
   if (M < kDenseTokens || cus <= 0) return false;
+  // The SwiGLU forms give the bits of the plain GEMM and the elementwise kernel: they choose a
+  // route of their own only where both routes run the reduction whole, and so add in one order.
+  if (glu) {
+    int cfg, sp;
+    choose(M, Nc, Kr, bwd, &cfg, &sp);
+    const bool plain = dense_plan(M, Nc, Kr, bwd, false, d);
+    if (sp > 1 || (plain && d->splits > 1)) return plain;
+  }
   return dense_memo({{kPlanDense, cus, M, Nc, Kr, bwd, glu}}, d, [&](DensePlan* p) {
     const double f = fused_us(M, Nc, Kr, bwd, glu);
     if (f < 0) return false;
     const double t = dense_us(M, 1, &Nc, Kr / kBK, (int64_t)Nc * Kr, false, glu, 0, p);
-    return t > 0 && t < 0.97 * f;
+    return t > 0 && t < 0.97 * f && !(glu && p->splits > 1);
   });
 }
 
@@ -2693,11 +2701,20 @@ static int gemm_entry(bool bwd, const GemmArgs& a, int cfg, int splits, hipStrea
       if (rc != MXS_OK || a.glu != 1) return rc;
       return mxs_silu_mul(a.glu_g, a.C, a.glu_h, (int64_t)a.M * a.Nc, stream);
     }
-    DensePlan d;
-    if (a.ws && (uintptr_t)a.ws % 16 == 0 && a.glu != 1 && a.cols_blocks == 0 &&
-        dense_takes(a.M, a.Nc, a.Kr) && dense_plan(a.M, a.Nc, a.Kr, bwd, a.glu == 2, &d))
-      return launch_dense(bwd, &a, 1, false, d, a.ws, true, nullptr, stream);
     choose(a.M, a.Nc, a.Kr, bwd, &cfg, &splits);
+    DensePlan d;
+    if (a.ws && (uintptr_t)a.ws % 16 == 0 && a.cols_blocks == 0 &&
+        dense_takes(a.M, a.Nc, a.Kr) && dense_plan(a.M, a.Nc, a.Kr, bwd, a.glu == 2, &d)) {
+      if (a.glu != 1) return launch_dense(bwd, &a, 1, false, d, a.ws, true, nullptr, stream);
+      // the SwiGLU forward: the fused kernel, but where the sums would be in another order
+      if (splits > 1 || d.splits > 1) {
+        GemmArgs plain = a;
+        plain.glu = 0;
+        const int rc = launch_dense(false, &plain, 1, false, d, a.ws, true, nullptr, stream);
+        return rc != MXS_OK
+            ? rc : mxs_silu_mul(a.glu_g, a.C, a.glu_h, (int64_t)a.M * a.Nc, stream);
+      }
+    }
     // no workspace for a split of few tokens: the shape's own plan, where that has none
     if (splits > 1 && !a.ws) choose_base(a.M, a.Nc, a.Kr, bwd, &cfg, &splits);
   }
