@@ -2434,14 +2434,18 @@ struct DensePlan {
   int bn, splits;
 };
 
-// What the dense route and the fused kernels cost, in microseconds on MI355X (HIP graphs, M = 1024
-// to 8192, the projections' shapes): rounds of tiles over the CUs times a tile's time, which is a
-// K-step's time (power-limited when every CU multiplies) plus what stands alone at its ends.  The
-// route is taken where its estimate is 3 % below the fused kernels'.  Measured / estimated, dense
-// against fused: down_proj forward at 8192 tokens 220 / 228 against 370, at 3001 105 / 104 against
-// 128, at 2048 80 / 79 against 88; its dX (8960 wide) 244 / 247 against 267 at 8192, 68 / 66
-// against 75 at 2048, not taken at 3001 (113 / 129 against 112); 1536 x 1536 at 8192 49 / 47
-// against 66, not taken at 4096 (39 against 39).
+// What the dense route and the fused kernels cost, in microseconds on MI355X (HIP graphs replayed
+// in turn, 769 to 10240 tokens, the projections' shapes and those of hidden 2048 and 4096): rounds
+// of tiles over the CUs times a tile's time, which is a K-step's time (power-limited when every CU
+// multiplies) plus what stands alone at its ends.  Over 1500 such pairs the route chosen by the
+// estimates (dense_worth) takes 0.4 % more than the faster one on average.  Measured (estimated),
+// dense against fused:
+//   down_proj forward, 2048 tokens 84 (78) / 90 (89); 3001 106 (104) / 129 (133); 8192 230 (208)
+//   / 366 (352)
+//   its dX, 8960 wide, 2048 67 (65) / 75 (72); 3001 100 (104) / 110 (108); 8192 243 (229)
+//   / 269 (260)
+//   with the SwiGLU adjoint, 3001 121 (126) / 134 (130); 8192 357 (337) / 340 (340): not taken
+//   1536 x 1536, 4096 39 (45) / 40 (39): not taken; 8192 51 (48) / 67 (63)
 static double fused_tile_us(int cfg, int steps) {
   switch (cfg) {
     case 6: return 0.95 * steps + 7.0;             // 256x128
@@ -2452,9 +2456,20 @@ static double fused_tile_us(int cfg, int steps) {
   }
 }
 
-static double dense_tile_us(int bn, int steps) {
+// `ends`: what stands alone at a tile's ends, kDenseEnds and more for the kinds of tile below.
+static double dense_tile_us(int bn, int steps, double ends) {
   const double step = bn == 320 ? 1.78 : bn == 256 ? 1.47 : 1.32;
-  return step * steps + 13.0;
+  return step * steps + ends;
+}
+constexpr double kDenseEnds = 13.0;
+constexpr double kDenseEndsSum = 26.0;   // every problem's LoRA term and mask, one after the other
+constexpr double kDenseEndsRope = 21.0;  // the cos / sin rows, read when every tile is at its end
+
+// Whether a dense estimate is taken over the fused one: by 3 %, or by 6 % where the reduction is
+// split (the reduce's traffic is the least certain part: 4096 x 4096 at 1280 tokens, three splits,
+// was estimated 3 % better and measured 10 % worse).
+static bool dense_worth(double dense, double fused, const DensePlan& d) {
+  return dense > 0 && dense < (d.splits > 1 ? 0.94 : 0.97) * fused;
 }
 
 // `wgs` workgroups of t microseconds on the CUs; the last, partial round runs with idle CUs: an
@@ -2491,23 +2506,24 @@ static double fused_us(int M, int Nc, int Kr, bool bwd, bool glu) {
 }
 
 // The best dense plan for n problems [M, Nc[i]] over `steps` K-steps (sum: one output Nc[0] and
-// all problems' steps together), `values` weight values to decode; its time, or a negative
-// number if there is none.  `bn`: only this tile width (0: any).
+// all problems' steps together; rope: rotated), `values` weight values to decode; its time, or a
+// negative number if there is none.
 static double dense_us(int M, int n, const int* Nc, int steps, int64_t values, bool sum, bool glu,
-                       int bn, DensePlan* d) {
+                       bool rope, DensePlan* d) {
   const int cus = cu_count();
   if (cus <= 0 || M <= 0 || steps <= 0) return -1.0;
   const int64_t gy = ceil_div(M, kDenseBM);
   double best = -1.0;
   for (int w : {320, 256, 192}) {
-    if (bn ? w != bn : (sum && w != 192)) continue;  // summed tiles: 192 (registers)
+    if ((rope && w != 256) || (sum && w != 192)) continue;  // a wave per head; registers
     int64_t tiles = 0;
     for (int i = 0; i < (sum ? 1 : n); i++) tiles += gy * ceil_div(Nc[i], w);
     for (int sp = 1; sp <= 8; sp++) {
       if (sp > 1 && (w == 320 || (n > 1 && !sum) || steps / sp < 12)) break;
       const int per = (int)ceil_div(steps, sp);
       if (ceil_div(steps, per) != sp) continue;
-      const double t = rounds_us(tiles * sp, cus, dense_tile_us(w, per), kDenseAlone) +
+      const double ends = sum ? kDenseEndsSum : rope ? kDenseEndsRope : kDenseEnds;
+      const double t = rounds_us(tiles * sp, cus, dense_tile_us(w, per, ends), kDenseAlone) +
                        (glu ? glu_us(M, Nc[0], true) : 0.0) + reduce_us(sp, M, Nc[0]) +
                        2.53 * values / 4.2e6 + 1.5;
       if (best < 0 || t < best) {
@@ -2551,8 +2567,8 @@ static bool dense_plan(int M, int Nc, int Kr, bool bwd, bool glu, DensePlan* d) 
   return dense_memo({{kPlanDense, cus, M, Nc, Kr, bwd, glu}}, d, [&](DensePlan* p) {
     const double f = fused_us(M, Nc, Kr, bwd, glu);
     if (f < 0) return false;
-    const double t = dense_us(M, 1, &Nc, Kr / kBK, (int64_t)Nc * Kr, false, glu, 0, p);
-    return t > 0 && t < 0.97 * f && !(glu && p->splits > 1);
+    const double t = dense_us(M, 1, &Nc, Kr / kBK, (int64_t)Nc * Kr, false, glu, false, p);
+    return dense_worth(t, f, *p) && !(glu && p->splits > 1);
   });
 }
 
@@ -3183,9 +3199,10 @@ static int64_t dense_sum_bytes(int n, int M, const int* N, int K, const DensePla
   return 2 * weight_values(n, N, K) + planes;
 }
 
-// The gate / up pair's summed dX (against its split-K launch on 256x96 tiles).  Measured at 8192
-// tokens: 469 us and 19 us of decode against 613 us and a reduce of four planes; at 3001 tokens
-// 192 + 17 (and a reduce of two planes instead of four) against 212.
+// The gate / up pair's summed dX (against its split-K launch on 256x96 tiles).  Measured
+// (estimated) with decode and reduce: 1100 tokens 111 (116) / 124 (133) us; 2048 156 (149) / 152
+// (150) and 3001 230 (233) / 223 (224), not taken; 4096 287 (243) / 306 (299); 8192 498 (414) / 635
+// (595).
 static bool dense_pair_plan(int M, const int N[2], int K, DensePlan* d) {
   const int cus = cu_count();
   if (cus <= 0 || M < kDenseTokens || !dense_takes_all(2, M, N, K, true)) return false;
@@ -3199,8 +3216,9 @@ static bool dense_pair_plan(int M, const int N[2], int K, DensePlan* d) {
     const double f = rounds_us(ceil_div(M, 256) * ceil_div(K, 96) * 2 * sp, cus,
                                fused_tile_us(11, (int)ceil_div(longest, sp)), kFusedAlone) +
                      reduce_us(2 * sp, M, K);
-    const double t = dense_us(M, 2, &K, steps, weight_values(2, N, K), true, false, 0, p);
-    return t > 0 && t < 0.97 * f;
+    const double t = dense_us(M, 2, &K, steps, weight_values(2, N, K), true, false, false,
+                              p);
+    return dense_worth(t, f, *p);
   });
 }
 
@@ -3227,8 +3245,9 @@ static bool pair_plan(int M, const int N[2], int K, bool mixed_masks, const void
   return p->dense || pair_planes_bytes(M, K, p->splits) <= bytes;
 }
 
-// q, k and v's summed dX without their gradients (against one launch of 128x128 tiles): 84 us
-// and 5 us of decode against 110 at 8192 tokens.
+// q, k and v's summed dX without their gradients (against one launch of 128x128 tiles), measured
+// (estimated): 4096 tokens 71 (64) / 66 (63) us, not taken; 6144 75 (69) / 97 (95); 8192 88 (72) /
+// 106 (101).
 static bool dense_sum_plan(int n, int M, const int* N, int K, DensePlan* d) {
   const int cus = cu_count();
   if (cus <= 0 || M < kDenseTokens || n < 2 || n > kMaxSum || !dense_takes_all(n, M, N, K, true))
@@ -3239,15 +3258,16 @@ static bool dense_sum_plan(int n, int M, const int* N, int K, DensePlan* d) {
     for (int i = 0; i < n; i++) steps += N[i] / kBK;
     const double f = rounds_us(ceil_div(M, 128) * ceil_div(K, 128), cus,
                                fused_tile_us(10, steps) + 8.0, kFusedAlone);
-    const double t = dense_us(M, n, &K, steps, weight_values(n, N, K), true, false, 0, p);
-    return t > 0 && t < 0.97 * f;
+    const double t = dense_us(M, n, &K, steps, weight_values(n, N, K), true, false, false,
+                              p);
+    return dense_worth(t, f, *p);
   });
 }
 
-// Several forwards over one input in one launch: q, k and v (against 128x128 tiles; 70 us, rotated,
-// and 5 us of decode against 108 at 8192 tokens), or wide outputs (gate and up, against 256x160
-// tiles of which a mixed launch saves 5 %; 448 + 15 against 527 us at 8192, 164 + 14 against 209
-// at 3001).
+// Several forwards over one input in one launch, measured (estimated): q, k and v, rotated (against
+// 128x128 tiles), 4096 tokens 60 (56) / 54 (53) us, not taken, 6144 65 (58) / 80 (79), 8192 74 (60) /
+// 104 (106); wide outputs (gate and up, against 256x160 tiles of which a mixed launch saves 5 %),
+// 2048 tokens 125 (128) / 137 (137), 3001 178 (183) / 202 (205), 8192 448 (408) / 512 (495).
 static bool dense_group_plan(int n, int M, const int* N, int K, bool rope, DensePlan* d) {
   const int cus = cu_count();
   if (cus <= 0 || M < kDenseTokens || n < 1 || n > kMaxGemmGroup ||
@@ -3267,9 +3287,8 @@ static bool dense_group_plan(int n, int M, const int* N, int K, bool rope, Dense
     const double f = wide && !rope
         ? 0.95 * rounds_us(tiles160, cus, fused_tile_us(7, steps), kFusedAlone)
         : rounds_us(tiles128, cus, fused_tile_us(10, steps) + (rope ? 5.5 : 0.0), kFusedAlone);
-    const double t = dense_us(M, n, N, steps, weight_values(n, N, K), false, false, rope ? 256 : 0,
-                              p);
-    return t > 0 && t < 0.97 * f;
+    const double t = dense_us(M, n, N, steps, weight_values(n, N, K), false, false, rope, p);
+    return dense_worth(t, f, *p);
   });
 }
 
