@@ -95,13 +95,27 @@ int mxs_nf4_quantize(const void* w_f16, int64_t n_values, const float* code, voi
 
 /* ---- Fused NF4 GEMMs (forward and input gradient of the frozen Linear4bit) ---------------
  * cfg: tile configuration id (0-4: all-wave kernels, 6-12: producer/consumer kernels; 5 is
- * invalid) or -1 to let the library choose tiles and split-K for the shape; splits: reduction
- * splits (used with cfg >= 0).  When the plan splits the reduction, `workspace` must hold
- * mxs_nf4_gemm_workspace_bytes(M, Nc, Kr, cfg, splits) bytes of device memory (fp32 partial
- * sums, no initial contents needed; a return of 0 means no workspace is needed) and a second
- * small kernel adds the partials in split order: results are deterministic.  Shapes:
- * in_features % 64 == 0, reduction % 64 == 0; x/dy 16-byte aligned. */
+ * invalid) or -1 to let the library choose for the shape; splits: reduction splits (used with
+ * cfg >= 0).  workspace: device memory, no initial contents needed, of at least
+ * mxs_nf4_gemm_workspace_bytes(M, Nc, Kr, cfg, splits) bytes (0: none is used; with cfg -1 the
+ * most that either direction of the GEMM takes).  It holds fp32 partial sums where the plan splits
+ * the reduction (a second small kernel adds them in split order: results are deterministic) and,
+ * with cfg -1 at many tokens, the weight decoded to fp16 (mxs_nf4_linear_route).  With cfg -1
+ *   - a workspace that is given must hold those bytes whatever the plan: its presence alone lets
+ *     the plan use it;
+ *   - a NULL workspace is taken wherever some plan of the shape needs none (it then runs), and the
+ *     decoded weight also needs 16-byte alignment: without it the fused plan runs.
+ * The plans of one call may add the fp32 sums in different orders.  Shapes: in_features % 64 == 0,
+ * reduction % 64 == 0; x/dy 16-byte aligned. */
 int64_t mxs_nf4_gemm_workspace_bytes(int M, int Nc, int Kr, int cfg, int splits);
+
+/* Which kernels a planned call (cfg -1, aligned workspace) of a projection [K -> N0] at M tokens
+ * runs on the current device: 0 the fused ones, which decode the weight tile by tile, 1 the weight
+ * decoded once into the workspace and a plain fp16 GEMM, 2 the few-token kernel.  op: 0 forward, 1
+ * input gradient, 2 input gradient with the SwiGLU adjoint.  N1 > 0: two projections [K -> N0] and
+ * [K -> N1] in one call (op 0: mxs_nf4_linear_fwd_hp_pair or, for 1,
+ * mxs_nf4_linear_fwd_hp_group_ws; op 1: mxs_nf4_linear_bwd_dx_hp_pair).  MXS_ERR_ARG otherwise. */
+int mxs_nf4_linear_route(int op, int M, int N0, int N1, int K);
 
 /* Y[M,N] = X[M,K] . W[N,K]^T (+ bias[N]) (+ lora_h[M,r] . lora_b[N,r]^T), fp16 in/out, fp32
  * accumulation, W decoded from NF4 inside the GEMM.  Replaces NF4LinearFunction.forward
@@ -205,7 +219,8 @@ int mxs_nf4_linear_bwd_dx_hp(const void* dy, int M, int N, int K, const void* pa
  * plain GEMM runs the two reductions into one accumulator (split over a few planes where the
  * tiles are few).  Either way neither dX_i is rounded to fp16 on its own; the result equals the
  * fp32 sum of the two GEMMs rounded once.  Arrays hold the per-projection arguments (N[i] =
- * out_features; mask and lora_dht may be NULL, or any entry); the two share M, K, r, ldt,
+ * out_features; mask and lora_dht may be NULL, or any entry; a mask on one projection only keeps
+ * the split-K launch); the two share M, K, r, ldt,
  * hp_slices and mask_scale.  workspace: at least
  * mxs_nf4_linear_bwd_dx_pair_workspace_bytes(M, N[0], N[1], K) bytes (the decoded weights are
  * used only where it is 16-byte aligned).  Only where

@@ -3396,7 +3396,7 @@ static bool dx_grads_group_ok(int n, int M, const int* N, int K, int r, int* nw)
 
 using namespace mxs;
 
-// Split-K workspace: one fp32 partial plane per split.
+// One fp32 partial plane per split and, for the planned call, the decoded weight.
 int64_t mxs_nf4_gemm_workspace_bytes(int M, int Nc, int Kr, int cfg, int splits) {
   if (cfg >= 0)
     return splits > 1 ? (int64_t)splits * M * Nc * (int64_t)sizeof(float) : 0;
@@ -3417,6 +3417,18 @@ int64_t mxs_nf4_gemm_workspace_bytes(int M, int Nc, int Kr, int cfg, int splits)
     return {need, 0, 0};
   });
   return v[0];
+}
+
+int mxs_nf4_linear_route(int op, int M, int N0, int N1, int K) {
+  if (op < 0 || op > 2 || M <= 0 || N0 <= 0 || N1 < 0 || K <= 0 || (N1 > 0 && op > 1))
+    return MXS_ERR_ARG;
+  if (op == 0 && skinny_takes(M, N0, K)) return 2;
+  DensePlan d;
+  const int N[2] = {N0, N1};
+  if (N1 > 0)
+    return (op == 0 ? dense_group_plan(2, M, N, K, false, &d) : dense_pair_plan(M, N, K, &d)) ? 1 : 0;
+  const int Nc = op ? K : N0, Kr = op ? N0 : K;
+  return dense_takes(M, Nc, Kr) && dense_plan(M, Nc, Kr, op > 0, op > 1, &d) ? 1 : 0;
 }
 
 static void set_workspace(GemmArgs& a, void* workspace) {

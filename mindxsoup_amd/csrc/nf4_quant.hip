@@ -219,7 +219,8 @@ int mxs_nf4_quantize(const void* w_f16, int64_t n_values, const float* code, voi
     hipLaunchKernelGGL(k_absmax_mean, dim3(1), dim3(64), 0, stream, partial, (int)n_partial,
                        n_blocks, offset);
   hipLaunchKernelGGL(k_quant_absmax, dim3((unsigned)n_groups), dim3(256), 0, stream, absmax_f32,
-                     n_blocks, partial, here ? (int)n_partial : 0, offset, code, static_cast<uint8_t*>(absmax8), absmax2);
+                     n_blocks, partial, here ? (int)n_partial : 0, offset, code,
+                     static_cast<uint8_t*>(absmax8), absmax2);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? MXS_OK : (int)e;
 }

@@ -112,7 +112,8 @@ __global__ __launch_bounds__(64 * (kSkinnyWaves + 1)) void k_nf4_skinny(SkinnyGr
         }
       }
     }
-  } else if (wave == lw) {  // bias + LoRA, and the transposed LoRA operand from the first columns' workgroup
+  } else if (wave == lw) {
+    // bias + LoRA, and the transposed LoRA operand from the first columns' workgroup
     if (a.bias) {
       const float bv = (float)a.bias[n];
       acc = (float4_t){bv, bv, bv, bv};

@@ -5,7 +5,8 @@ allocator, and launches on the current HIP stream.  Nothing here computes on the
 back to another implementation: an unsupported shape raises.
 
 Workspaces: the split-K GEMMs write fp32 partial sums to a workspace that a second small kernel
-adds up in a fixed order; its contents need no initialisation and are dead after the call, so
+adds up in a fixed order, and at many tokens the weight is decoded to fp16 there (2 bytes a value:
+28 MB for 8960 x 1536); its contents need no initialisation and are dead after the call, so
 one buffer serves any number of calls issued in order on one stream.  Calls take it as `ws` or
 allocate it from torch's caching allocator.  The LoRA H / dH kernels use one the same way for
 reductions of 1024 or more (split over workgroups); the dA / dB kernel needs none.
@@ -115,6 +116,16 @@ def fused_shape_ok(state, M=None):
 
 def gemm_workspace_bytes(M, Nc, Kr, cfg=-1, splits=1):
     return int(_lib.lib().mxs_nf4_gemm_workspace_bytes(M, Nc, Kr, cfg, splits))
+
+
+def gemm_route(op, M, N, K, N1=0):
+    """"fused", "dense" (weight decoded once into the workspace) or "few": the kernels of a planned
+    call of a projection K -> N at M tokens, op "fwd", "dx" or "dx_glu"; with N1 the two projections
+    K -> N and K -> N1 in one call (mxs_nf4_linear_route)."""
+    rc = _lib.lib().mxs_nf4_linear_route(("fwd", "dx", "dx_glu").index(op), M, N, N1, K)
+    if rc < 0:
+        _lib.check(rc, "mxs_nf4_linear_route")
+    return ("fused", "dense", "few")[rc]
 
 
 def lora_workspace_bytes(M, K, N, r):

@@ -23,7 +23,8 @@ def _proj(dev, n, M, r, seed):
     rnd = lambda *s: torch.randn(s, device=dev, generator=g)  # noqa: E731
     packed, st = quantize_4bit((rnd(n, K) * 0.02).half())
     return dict(n=n, packed=packed, st=st, a=(rnd(r, K) / K ** 0.5).half(),
-                b=(rnd(n, r) * 0.01).half(), dy=rnd(M, n).half(), ht=rnd(r, (M + 7) // 8 * 8).half(),
+                b=(rnd(n, r) * 0.01).half(), dy=rnd(M, n).half(),
+                ht=rnd(r, (M + 7) // 8 * 8).half(),
                 keep=(torch.rand((M, K), device=dev, generator=g) >= 0.05).to(torch.uint8))
 
 
@@ -36,13 +37,13 @@ def _bound(parts, two):
 @pytest.mark.parametrize("r", [16, 32, 64])
 @pytest.mark.parametrize("masked", [(True, False), (False, True), (False, False), (True, True)])
 def test_masks_of_either_projection(cuda, masked, r, widths):
-    from mindxsoup_amd import _lib, kernels
+    from mindxsoup_amd import kernels
 
     M = 1430  # the last row band holds 150 rows
     print(f"case dense dX pair masked={masked} r={r} widths={widths}", flush=True)
-    nbytes = _lib.lib().mxs_nf4_linear_bwd_dx_pair_workspace_bytes(M, *widths, K)
-    if nbytes < 2 * sum(widths) * K:  # room for the decoded weights: the dense route
-        pytest.skip("this device's CU count plans the fused kernel")
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the plans of another CU count")
+    assert kernels.gemm_route("dx", M, widths[0], K, widths[1]) == "dense"
     ps = [_proj(cuda, n, M, r, 20 + i) for i, n in enumerate(widths)]
     keeps = [p["keep"] if m else None for p, m in zip(ps, masked)]
     dhps = [kernels.lora_dh_partials(p["dy"], p["b"].t().contiguous(), S) for p in ps]
@@ -68,7 +69,7 @@ def test_masks_of_either_projection(cuda, masked, r, widths):
         assert torch.equal(da, da1) and torch.equal(db, db1)
 
 
-@pytest.mark.parametrize("M", [64, 1430, 3001, 8192])
+@pytest.mark.parametrize("M", [64, 1430, 3001, 3200, 8192])
 def test_callers_workspace(cuda, M):
     """A workspace of projection_workspace_bytes serves the summed gradient at every token count,
     whatever the faster plan would take (more fp32 planes at few tokens, the decoded weights at

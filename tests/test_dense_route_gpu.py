@@ -29,6 +29,15 @@ def _proj(dev, n, k, M, r, seed, x=None, bias=False):
                 keep=(torch.rand((M, k), device=dev, generator=g) >= 0.05).to(torch.uint8))
 
 
+def _on_dense_route(op, M, n, k, n1=0):
+    """The planned call runs on decoded weights (else, on another CU count, the test is skipped)."""
+    from mindxsoup_amd import kernels
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the plans of another CU count")
+    assert kernels.gemm_route(op, M, n, k, n1) == "dense"
+
+
 def _close(got, want):
     d = (got.float() - want.float()).abs()
     bound = 2.0 ** -10 * want.float().abs() + 2.0 ** -20 * want.float().abs().max()
@@ -53,8 +62,7 @@ def test_forward(cuda, n, k, M, r, bias, splits):
 
     print(f"case dense fwd n={n} k={k} M={M} r={r}", flush=True)
     p = _proj(cuda, n, k, M, r, 1, bias=bias)
-    if kernels.gemm_workspace_bytes(M, n, k) < 2 * n * k:
-        pytest.skip("this device's CU count plans the fused kernel")
+    _on_dense_route("fwd", M, n, k)
     hp, _, _ = kernels.lora_h_partials(p["x"], p["a"], S, p["keep"], MS, lora_b=p["b"])
     y, ht = kernels.nf4_linear_fwd_hp(p["x"], p["packed"], p["st"], hp, p["b"], p["bias"])
     y0, ht0 = kernels.nf4_linear_fwd_hp(p["x"], p["packed"], p["st"], hp, p["b"], p["bias"],
@@ -77,8 +85,7 @@ def test_input_gradient(cuda, n, k, M, r, masked, split):
 
     print(f"case dense dx n={n} k={k} M={M} r={r}", flush=True)
     p = _proj(cuda, n, k, M, r, 2)
-    if kernels.gemm_workspace_bytes(M, k, n) < 2 * n * k:
-        pytest.skip("this device's CU count plans the fused kernel")
+    _on_dense_route("dx", M, n, k)
     keep = p["keep"] if masked else None
     dhp = kernels.lora_dh_partials(p["dy"], p["b"].t().contiguous(), S)
     at = p["a"].t().contiguous()
@@ -140,13 +147,18 @@ def test_qkv_group_with_rope_and_summed_dx(cuda, M, T, r):
     assert bool(((dx.float() - two).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("M", [1430, 3001, 8192])
-def test_gate_up_pair(cuda, M):
-    """gate and up: forward in one dense launch where planned (the bits of two), the summed dX
-    (several splits, and unsplit at 8192) and both projections' gradients."""
+# which of the two is on decoded weights: the summed dX in five splits, the forward, both (two
+# splits, and unsplit)
+@pytest.mark.parametrize("M,dense", [(1430, ("dx",)), (3001, ("fwd",)), (3200, ("fwd", "dx")),
+                                     (8192, ("fwd", "dx"))])
+def test_gate_up_pair(cuda, M, dense):
+    """gate and up: forward in one launch (the bits of two), the summed dX and both projections'
+    gradients."""
     from mindxsoup_amd import kernels
 
     print(f"case dense pair M={M}", flush=True)
+    for op in dense:
+        _on_dense_route(op, M, 8960, 1536, 8960)
     x = torch.randn((M, 1536), device=cuda).half()
     ps = [_proj(cuda, 8960, 1536, M, 16, 9 + i, x=x) for i in range(2)]
     rows = kernels.lora_h_partials_group([x] * 2, [p["a"] for p in ps], S,
@@ -175,3 +187,38 @@ def test_gate_up_pair(cuda, M):
     bound = 2.0 ** -11 * (sum(t.float().abs() for t in parts) + two.abs()) * 1.01 + \
         2.0 ** -18 * two.abs().max()  # and the fp32 sums' other order
     assert bool(((dx.float() - two).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("op,n,k,n1", [("fwd", 1536, 8960, 0), ("fwd", 8960, 1536, 0),
+                                       ("dx", 1536, 8960, 0), ("dx", 8960, 1536, 0),
+                                       ("dx", 8960, 1536, 8960)])
+def test_first_planned_token_count(cuda, op, n, k, n1):
+    """The fewest tokens that decode the weight, and one fewer: within the split sums' bound."""
+    from mindxsoup_amd import kernels
+
+    first = next((M for M in range(2, 8192) if kernels.gemm_route(op, M, n, k, n1) == "dense"), 0)
+    if not first:
+        pytest.skip("the plans of another CU count")
+    print(f"case first dense {op} n={n} k={k} n1={n1} M={first}", flush=True)
+    for M in (first, first - 1):
+        ps = [_proj(cuda, n, k, M, 16, 40 + i) for i in range(2 if n1 else 1)]
+        if op == "fwd":
+            args = (ps[0]["x"], ps[0]["packed"], ps[0]["st"])
+            _close(kernels.nf4_linear_fwd(*args), kernels.nf4_linear_fwd(*args, cfg=10, splits=1))
+            continue
+        dhps = [kernels.lora_dh_partials(p["dy"], p["b"].t().contiguous(), S) for p in ps]
+        ats = [p["a"].t().contiguous() for p in ps]
+        parts = [kernels.nf4_linear_bwd_dx_hp(p["dy"], p["packed"], p["st"], h, at, p["keep"], MS,
+                                              cfg=10, splits=1)[0]
+                 for p, h, at in zip(ps, dhps, ats)]
+        if not n1:
+            _close(kernels.nf4_linear_bwd_dx_hp(ps[0]["dy"], ps[0]["packed"], ps[0]["st"], dhps[0],
+                                                ats[0], ps[0]["keep"], MS)[0], parts[0])
+            continue
+        dx, _ = kernels.nf4_linear_bwd_dx_hp_pair(
+            [p["dy"] for p in ps], [p["packed"] for p in ps], [p["st"] for p in ps], dhps, ats,
+            [p["keep"] for p in ps], MS)
+        two = parts[0].float() + parts[1].float()
+        bound = 2.0 ** -11 * (sum(t.float().abs() for t in parts) + two.abs()) * 1.01 + \
+            2.0 ** -18 * two.abs().max()
+        assert bool(((dx.float() - two).abs() <= bound).all())

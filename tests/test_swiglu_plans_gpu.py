@@ -1,6 +1,6 @@
 """The SwiGLU forms of a GEMM (mxs_nf4_linear_fwd_glu, mxs_nf4_linear_bwd_dx_glu) against the plain
-GEMM and the elementwise kernel at many tokens, at shapes where decoding the weight pays for one form
-and not for the other, or splits the reduction in one and not the other: the same bits."""
+GEMM and the elementwise kernel at many tokens, at shapes where decoding the weight pays for one
+form and not for the other, or splits the reduction in one and not the other: the same bits."""
 
 import pytest
 import torch
