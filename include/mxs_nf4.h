@@ -220,8 +220,7 @@ int mxs_nf4_linear_bwd_dx_hp(const void* dy, int M, int N, int K, const void* pa
  * tiles are few).  Either way neither dX_i is rounded to fp16 on its own; the result equals the
  * fp32 sum of the two GEMMs rounded once.  Arrays hold the per-projection arguments (N[i] =
  * out_features; mask and lora_dht may be NULL, or any entry; a mask on one projection only keeps
- * the split-K launch); the two share M, K, r, ldt,
- * hp_slices and mask_scale.  workspace: at least
+ * the split-K launch); the two share M, K, r, ldt, hp_slices and mask_scale.  workspace: at least
  * mxs_nf4_linear_bwd_dx_pair_workspace_bytes(M, N[0], N[1], K) bytes (the decoded weights are
  * used only where it is 16-byte aligned).  Only where
  * mxs_nf4_linear_bwd_dx_pair_ok(M, N[0], N[1], K) is 1 (both projections plan the narrow-output
@@ -461,7 +460,8 @@ int mxs_nf4_linear_fwd_hp_group(int n, const void* const x[], int M, int K, cons
  * at b * cos_stride_b + t * cos_stride_t, cos_stride_b may be 0; 16-byte aligned, strides
  * multiples of 4).  At every token count the stored fp16 has the bits of
  * mxs_nf4_linear_fwd_hp_group followed by mxs_qkv_rope (forward, no LoRA term) on those outputs;
- * the remaining outputs (v) are unchanged.  N[i] of a rotated output: a multiple of 128; M a multiple of n_tokens. */
+ * the remaining outputs (v) are unchanged.  N[i] of a rotated output: a multiple of 128; M a
+ * multiple of n_tokens. */
 int mxs_nf4_linear_fwd_hp_group_rope(int n, const void* const x[], int M, int K, const int N[],
                                      const void* const packed[], const void* const absmax8[],
                                      const float* const code[], const float* const absmax2[],

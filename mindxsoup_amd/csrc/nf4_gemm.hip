@@ -2357,7 +2357,10 @@ static double few_us(int cus, int cfg, int sp, int M, int Nc, int steps) {
 
 // The planned configuration.  At up to 768 tokens the shapes' plans above leave most CUs idle (one
 // or two row bands: gate_proj 56 tiles of 256x160 at 256 tokens, down_proj 64 workgroups), and the
-// tile and split with the smallest estimate are taken where it is 8 % below the base plan's.
+// tile and split with the smallest estimate are taken where it is 8 % below the base plan's.  Past
+// 512 tokens more splits than the base plan's are charged 15 % more: most CUs are busy then, and
+// the tile times and the reduce come out longer (down forward on seven splits instead of four was
+// estimated 10 % faster at 700 and 768 tokens and measured 4 and 10 % slower).
 // Measured, planned / base: gate forward 12.8 / 24.9 us at 64 tokens, 18.6 / 25.4 at 200, 20.1 /
 // 26.1 at 300, 28.1 / 32.8 at 700; down forward 15.0 / 27.4, 20.5 / 31.7, 24.8 / 33.0; a
 // 4096 x 11008 projection (wide and long: one split in the base plan) 24.6 / 57.3, 36.8 / 62.6,
@@ -2379,7 +2382,7 @@ static void choose(int M, int Nc, int Kr, bool bwd, int* cfg, int* splits) {
              (sp > base_sp && (int64_t)sp * M * Nc * 4 > (int64_t)MXS_NF4_SCRATCH_BYTES)))
           break;
         if (ceil_div(steps, ceil_div(steps, sp)) != sp) continue;
-        const double t = few_us(cus, c, sp, M, Nc, steps);
+        const double t = few_us(cus, c, sp, M, Nc, steps) * (M > 512 && sp > base_sp ? 1.15 : 1.0);
         if (t < best) {
           best = t;
           best_c = c;
